@@ -288,6 +288,277 @@ static int launch_prefill_f32(const PrefillParams& prm, hipStream_t stream) {
     return check_launch("prefill_f32_kernel");
 }
 
+template <int N>
+__device__ __forceinline__ void wait_vm_n() {
+    static_assert(N == 0 || N == 8 || N == 16, "vmcnt immediates used by the fp32 kernels below");
+    if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    if constexpr (N == 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+}
+
+// ------------------------------------------------------------------------------------------------
+// Key-split form: a workgroup is 4 waves over the SAME 32 query rows, and wave w takes the key tiles
+// t = w, w + 4, ...; the waves' (O, max, row sum) meet in LDS at the end.  Against the 128-row form
+// above, a work item is a quarter of the rows and its serial chain of key tiles a quarter as long, so
+// a grid that fills the chip only once or less (where the longest causal item sets the time) ends
+// sooner; each K/V tile then feeds one wave instead of four, which the fp32 MFMAs leave room for (16
+// to 32 B/clk per CU of tile loads against ~64).
+//
+// Each wave loads its own tiles into its own LDS buffers, so the loop has no barrier.  The buffers are
+// single: K(t+4) lands while PV(t) runs and V(t+4) while S(t+4) runs (1,024 to 4,096 MFMA cycles each).
+template <int D, bool CAUSAL, bool MASKED, bool PAD>
+__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(const PrefillParams p) {
+    constexpr int NW = 4;
+    constexpr int BN = 32;           // keys per tile
+    constexpr int DCH = D / 4;       // 16-byte chunks per row
+    constexpr int HD = D / 2;        // S^T k-steps: dimensions per lane half
+    constexpr int DT = D / 32;       // 32-row d blocks of O^T
+    constexpr int RPI = 1024 / (4 * D);  // rows per 1 KB load instruction
+    constexpr int INSTR = BN / RPI;      // load instructions per tile (all by the tile's wave)
+    static_assert(D == 64 || D == 128, "head dim 64 or 128");
+    typedef float fvec __attribute__((ext_vector_type(DT)));
+
+    __shared__ __attribute__((aligned(16))) float tiles[NW][2][BN * D];  // K, V of each wave; then its O
+    __shared__ float red[2][NW][32];                                     // row maxima and sums of each wave
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31;
+    const int hf = lane >> 5;
+
+    const BlockCoord bc = block_coord<CAUSAL>(p);
+    const int b = bc.b, hq = bc.hq, hk = bc.hk;
+    const float* qp = reinterpret_cast<const float*>(p.q) + b * p.qs_b + hq * p.qs_h;
+    const float* kp = reinterpret_cast<const float*>(p.k) + b * p.ks_b + hk * p.ks_h;
+    const float* vp = reinterpret_cast<const float*>(p.v) + b * p.vs_b + hk * p.vs_h;
+
+    const int q0 = bc.qb * 32;
+    int kend = p.Sk;
+    if (CAUSAL) {
+        const int lim = q0 + 32 + p.delta;  // keys < lim can be visible
+        kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
+    }
+    const int nt = (kend + BN - 1) / BN;
+    const int krow = (int)(p.ks_s * (int64_t)sizeof(float));  // row pitch in bytes (host-checked)
+    const int vrow = (int)(p.vs_s * (int64_t)sizeof(float));
+    float* Kt = tiles[wave][0];
+    float* Vt = tiles[wave][1];
+
+    // Tile t -> this wave's buffer, as in the kernel above (slot c of row r holds chunk c ^ (r & 15); rows past
+    // Sk and, under PAD, chunks past valid_ch read zeros).
+    auto dma = [&](float* dst, const float* base, int pitch, int64_t stride, int t, int valid_ch) {
+        const int rows = min(BN, p.Sk - t * BN);
+        const uint32_t nbytes = (uint32_t)((rows - 1) * pitch + (PAD ? valid_ch * 16 : D * 4));
+        const auto rs = make_rsrc(base + (int64_t)t * BN * stride, nbytes);
+#pragma unroll
+        for (int i = 0; i < INSTR; ++i) {
+            const int r = i * RPI + lane / DCH;
+            const int c = (lane % DCH) ^ (r & 15);
+            const uint32_t off = (PAD && c >= valid_ch) ? 0x80000000u : (uint32_t)(r * pitch + c * 16);
+            buf_ld16_lds_async(rs, dst + i * RPI * D, off);
+        }
+    };
+
+    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
+    const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
+    const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(q0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
+
+    float qf[HD];
+    f32x16 oacc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+    float mrow = kNegInf, lrow = 0.f;
+
+    if (wave < nt) {
+        dma(Kt, kp, krow, p.ks_s, wave, p.qk_ch);
+        dma(Vt, vp, vrow, p.vs_s, wave, p.v_ch);
+    }
+    // Q as in the kernel above: lane (l32, hf) holds Q[q0 + l32][HD*hf + s], s < HD
+    {
+        const int qrow = q0 + l32;
+        const bool row_ok = qrow < p.Sq;
+        const float* qsrc = qp + (int64_t)(row_ok ? qrow : p.Sq - 1) * p.qs_s;
+#pragma unroll
+        for (int g = 0; g < HD / 4; ++g) {
+            const int ch = (HD / 4) * hf + g;
+            const bool ok = row_ok && (!PAD || ch < p.qk_ch);
+            const float* src = (!PAD || ch < p.qk_ch) ? qsrc + 4 * ch : qsrc;
+            const u32x4 raw = q_bits(ld16(src), ok ? p.q_and : 0u, ok ? p.q_xor : 0u);
+            const f32x4 x = __builtin_bit_cast(f32x4, raw);
+            qf[4 * g + 0] = x.x, qf[4 * g + 1] = x.y, qf[4 * g + 2] = x.z, qf[4 * g + 3] = x.w;
+        }
+    }
+    // Q and the first tile complete here, visibly to the compiler (no load waits of its own inside the loop)
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+
+    for (int t = wave; t < nt; t += NW) {
+        const int kbase = t * BN;
+        const bool more = t + NW < nt;
+        wait_vm_n<INSTR>();  // K(t) landed; V(t), issued after it, may be in flight
+        u32x4 mraw[4];
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) mraw[g] = buf_ld16(mrs, mrow_off + (uint32_t)((kbase + 8 * g + 4 * hf) * 4));
+        }
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.f;
+        {
+            const int r = l32;
+#pragma unroll
+            for (int g = 0; g < HD / 4; ++g) {
+                const int c = (HD / 4) * hf + g;
+                const f32x4 kv = *reinterpret_cast<const f32x4*>(Kt + r * D + 4 * (c ^ (r & 15)));
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qf[4 * g + 0], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qf[4 * g + 1], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qf[4 * g + 2], s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qf[4 * g + 3], s, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+            for (int g = 0; g < HD / 4 - 2; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+        }
+        // every K(t) read has returned: K(t+4) may land
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (more) dma(Kt, kp, krow, p.ks_s, t + NW, p.qk_ch);
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 m = __builtin_bit_cast(f32x4, mraw[g]);
+                s[4 * g + 0] += m.x * p.inv_scale;
+                s[4 * g + 1] += m.y * p.inv_scale;
+                s[4 * g + 2] += m.z * p.inv_scale;
+                s[4 * g + 3] += m.w * p.inv_scale;
+            }
+        }
+        const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && (kbase + BN - 1 > q0 + p.delta));
+        if (need_mask) {
+            int lim = p.Sk - 1 - kbase;
+            if (CAUSAL) lim = min(lim, q0 + l32 + p.delta - kbase);
+            lim -= 4 * hf;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (8 * (i >> 2) + (i & 3) > lim) s[i] = kNegInf;
+        }
+        float mx = kNegInf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        mx = max_xor32(mx);
+        const float mcand = fmaxf(mrow, mx * p.c);
+        if (__any(mcand - mrow > kRescaleThreshold)) {  // wave-uniform
+            const float alpha = fast_exp2(mrow - (mcand == kNegInf ? 0.f : mcand));
+            mrow = mcand;
+            lrow *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
+        }
+        const float mbase = (mrow == kNegInf) ? 0.f : mrow;
+        float pr[16];
+        float ls = lrow;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            pr[i] = fast_exp2(__builtin_fmaf(s[i], p.c, -mbase));
+            ls += pr[i];
+        }
+        lrow = ls;
+        // V(t) landed; the K(t+4) loads issued after it may be in flight
+        if (more)
+            wait_vm_n<INSTR>();
+        else
+            wait_vm_n<0>();
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int key = 8 * jj + 4 * hf + rr;
+                const int e = DT * l32;
+                const fvec vv = *reinterpret_cast<const fvec*>(Vt + key * D + 4 * ((e >> 2) ^ (key & 15)) + (e & 3));
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[dt], pr[4 * jj + rr], oacc[dt], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+        for (int i = 0; i < 14; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, DT, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * DT, 0);
+        // every V(t) read has returned: V(t+4) may land
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (more) dma(Vt, vp, vrow, p.vs_s, t + NW, p.v_ch);
+    }
+
+    // Merge: O of wave w, element i of block dt of lane l at (64 i + l) DT + dt of its K buffer (all of its
+    // loads have landed: the last tile waits for them).  Wave w then combines elements 4w .. 4w+3 of every
+    // wave by the row maxima: columns DT (8w + 4 hf + 0..3) of the output.
+    float* Ow = tiles[wave][0];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        fvec o;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = oacc[dt][i];
+        *reinterpret_cast<fvec*>(Ow + (64 * i + lane) * DT) = o;
+    }
+    const float lw = sum_xor32(lrow);
+    if (hf == 0) red[0][wave][l32] = mrow, red[1][wave][l32] = lw;
+    lds_barrier();
+    float M = kNegInf;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, red[0][w][l32]);
+    float f[NW], l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const float m = red[0][w][l32];
+        f[w] = m == kNegInf ? 0.f : fast_exp2(m - M);  // a max of -inf carries no keys
+        l = __builtin_fmaf(f[w], red[1][w][l32], l);
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int qrow = q0 + l32;
+    if (qrow < p.Sq) {
+        float* orow = reinterpret_cast<float*>(p.o) + b * p.os_b + hq * p.os_h + (int64_t)qrow * p.os_s;
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            fvec o;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const fvec x = *reinterpret_cast<const fvec*>(tiles[w][0] + (64 * (4 * wave + i4) + lane) * DT);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_fmaf(f[w], x[dt], o[dt]);
+            }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] *= inv;
+            const int col = DT * (8 * wave + 4 * hf + i4);
+            if (!PAD || col < 4 * p.v_ch) *reinterpret_cast<fvec*>(orow + col) = o;
+        }
+        if (p.lse != nullptr && hf == 0 && wave == 0)
+            p.lse[b * p.lses_b + hq * p.lses_h + qrow] = l > 0.f ? (M + __log2f(l)) * kLn2 : kNegInf;
+    }
+}
+
+template <int D, bool CAUSAL, bool MASKED, bool PAD>
+static int launch_prefill_f32_ks(const PrefillParams& prm, hipStream_t stream) {
+    PrefillParams p = prm;
+    p.n_qblocks = (p.Sq + 31) / 32;
+    const int64_t grid = (int64_t)p.n_qblocks * p.B * p.Hq;
+    if (grid == 0) return DTATTN_OK;
+    if (grid > 0x7fffffff) return fail(DTATTN_ERR_UNSUPPORTED, "prefill grid too large (%lld blocks)", (long long)grid);
+    hipLaunchKernelGGL((prefill_f32_ks_kernel<D, CAUSAL, MASKED, PAD>), dim3((unsigned)grid), dim3(256), 0, stream, p);
+    return check_launch("prefill_f32_ks_kernel");
+}
+
 // ------------------------------------------------------------------------------------------------
 // fp32 at kernel head dims 256 and 512 (the diffusers VAE attention, one head of 512, run in fp32).
 //
@@ -305,14 +576,6 @@ static int launch_prefill_f32(const PrefillParams& prm, hipStream_t stream) {
 // overlap the other half of the previous tile's work: 144 KB of LDS with the 16 KB exchange at D = 512.
 // Row i of the d-block dt of a wave's O^T is dimension w D/4 + DQ i + dt (DQ = D/128 blocks), so one
 // LDS read of DQ consecutive floats of a V row feeds the DQ MFMAs of a PV step, as in the kernel above.
-template <int N>
-__device__ __forceinline__ void wait_vm_n() {
-    static_assert(N == 0 || N == 8 || N == 16, "vmcnt immediates used by the wide fp32 kernel");
-    if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    if constexpr (N == 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-}
-
 template <int D, bool CAUSAL, bool MASKED, bool PAD>
 __global__ void __launch_bounds__(256, 1) prefill_f32_wide_kernel(const PrefillParams p) {
     constexpr int NW = 4;
@@ -571,8 +834,59 @@ static int launch_prefill_f32_wide(const PrefillParams& prm, hipStream_t stream)
     return check_launch("prefill_f32_wide_kernel");
 }
 
+// Whether the key-split form is expected to beat the 128-row form, on a model in units of one 32-key tile of a
+// whole workgroup (about 2.1 us a CU at D = 64, 4.0 us at D = 128).  A grid cannot end before its longest item,
+// nor before its work is spread over the CUs; a causal grid, longest items first, ends about a quarter of its
+// longest item after that.  At full load the key-split form costs 6% (D = 64) or 30% (D = 128: one workgroup
+// per CU) more per tile.  Measured, 128-row against key-split form, us (B x H x S):
+//   D = 64:  1x8x512 causal 38.5 / 13.1, 2x16x1000 causal 72.9 / 46.7, not causal 71.8 / 71.9, 1x12x2048
+//            137.6 / 102.8, 4x16x2048 causal 296 / 288, 4x32x2048 causal 548 / 591
+//   D = 128: 1x8x512 causal 70.2 / 24.5, 2x16x1000 causal 135 / 101, not causal 137 / 159, 1x12x2048 causal
+//            263 / 135, 4x16x1000 causal 185 / 199
+static bool f32_key_split(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
+    if (D != 64 && D != 128) return false;
+    int dev = 0;
+    dtattn_device_peaks pk;
+    if ((stream == nullptr ? hipGetDevice(&dev) : hipStreamGetDevice(stream, &dev)) != hipSuccess ||
+        dtattn_get_device_peaks(dev, &pk) != DTATTN_OK || pk.cu_count <= 0)
+        return false;
+    const int64_t heads = (int64_t)p.B * p.Hq, blocks = ((int64_t)p.Sq + 127) / 128, cus = pk.cu_count;
+    if (heads * blocks > 8 * cus) return false;  // many rounds: the 128-row form (and a bound on the sums below)
+    const double e = D == 64 ? 1.06 : 1.3;
+    // tiles of the rows of block i (rows each), and their sum over the blocks
+    auto tiles = [&](int64_t i, int64_t rows) {
+        const int64_t lim = causal ? (i + 1) * rows + p.delta : p.Sk;
+        const int64_t kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
+        return (kend + 31) / 32;
+    };
+    int64_t sum = 0, sum_ks = 0, longest = 0, longest_ks = 0;
+    for (int64_t i = 0; i < blocks; ++i) {
+        const int64_t t = tiles(i, 128);
+        sum += t;
+        longest = t > longest ? t : longest;
+    }
+    for (int64_t i = 0; i * 32 < p.Sq; ++i) {
+        const int64_t t = (tiles(i, 32) + 3) / 4;
+        sum_ks += t;
+        longest_ks = t > longest_ks ? t : longest_ks;
+    }
+    auto cost = [&](int64_t total, int64_t chain, int64_t items) {
+        if (!causal) return (double)((items + cus - 1) / cus) * (double)chain;
+        const double spread = (double)(total * heads) / (double)cus + 0.25 * (double)chain;
+        return spread > (double)chain ? spread : (double)chain;
+    };
+    return e * cost(sum_ks, longest_ks, heads * (((int64_t)p.Sq + 31) / 32)) < cost(sum, longest, heads * blocks);
+}
+
 template <bool MASKED, bool PAD>
 static int dispatch_prefill_f32_m(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
+    if (f32_key_split(p, D, causal, stream)) {
+        if (D == 128)
+            return causal ? launch_prefill_f32_ks<128, true, MASKED, PAD>(p, stream)
+                          : launch_prefill_f32_ks<128, false, MASKED, PAD>(p, stream);
+        return causal ? launch_prefill_f32_ks<64, true, MASKED, PAD>(p, stream)
+                      : launch_prefill_f32_ks<64, false, MASKED, PAD>(p, stream);
+    }
     if (D == 128)
         return causal ? launch_prefill_f32<128, true, MASKED, PAD>(p, stream)
                       : launch_prefill_f32<128, false, MASKED, PAD>(p, stream);
