@@ -27,12 +27,14 @@
 // PAD: the real head dims are below the kernel's D (any multiples of 4, Dv may differ from D), as in
 // the bf16 kernel: Q/K chunks past p.qk_ch and V chunks past p.v_ch load as zeros (adding nothing to
 // the scores, giving O columns that are never stored), and O chunks past p.v_ch are not written.
+#include <type_traits>
+
 #include "dtattn_common.hpp"
 #include "prefill_params.hpp"
 
 namespace dtattn {
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
+template <int D, bool CAUSAL, int MASKED, bool PAD>
 __global__ void __launch_bounds__(256, 2) prefill_f32_kernel(const PrefillParams p) {
     constexpr int NW = 4;
     constexpr int BN = 32;           // keys per tile
@@ -106,12 +108,11 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_kernel(const PrefillParams
         }
     };
 
-    // MASKED: lane (l32, hf) reads, for query row wq0 + l32, keys kbase + 8g + 4hf .. +3 (g < 4) of
-    // the (b, hq) mask slab, behind a buffer resource (reads past its last row return 0; those keys
-    // are hidden by the ragged-tail mask anyway).
-    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
-    const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
-    const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(wq0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
+    // MASKED: lane (l32, hf) reads, for query row wq0 + l32, keys kbase + 8g + 4hf .. +3 (g < 4).
+    const auto mslab = [&] {
+        if constexpr (MASKED != kMaskNone) return MaskSlab<MASKED>(p, b, hq, wq0 + l32);
+        else return 0;
+    }();
 
     auto tile = [&](const float* Kc, const float* Vc, float* Kn, float* Vn, int t) {
         wait_vmem();
@@ -122,17 +123,17 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_kernel(const PrefillParams
                 dma(Vn, vp, vrow, p.vs_s, t + 1, p.v_ch);
             }
         };
-        if constexpr (!MASKED) next_tile();
+        if constexpr (MASKED == kMaskNone) next_tile();
         const int kbase = t * BN;
         if (CAUSAL && kbase > wq0 + 31 + p.delta) {  // every row of this wave precedes the tile
-            if constexpr (MASKED) next_tile();
+            if constexpr (MASKED != kMaskNone) next_tile();
             return;
         }
         const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && (kbase + BN - 1 > wq0 + p.delta));
-        u32x4 mraw[4];
-        if constexpr (MASKED) {
+        typename MaskSlab<MASKED>::Group mraw[4];
+        if constexpr (MASKED != kMaskNone) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) mraw[g] = buf_ld16(mrs, mrow_off + (uint32_t)((kbase + 8 * g + 4 * hf) * 4));
+            for (int g = 0; g < 4; ++g) mraw[g] = mslab.load(kbase + 8 * g + 4 * hf);
         }
 
         // S^T = K Q^T: lane (l32, hf) supplies K[kbase + l32][HD*hf + s] at step s.
@@ -161,14 +162,12 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_kernel(const PrefillParams
             __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
         }
         // Element i of s holds key kbase + 8*(i/4) + 4*hf + i%4 of query wq0 + l32.
-        if constexpr (MASKED) {
+        if constexpr (MASKED != kMaskNone) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const f32x4 m = __builtin_bit_cast(f32x4, mraw[g]);
-                s[4 * g + 0] += m.x * p.inv_scale;
-                s[4 * g + 1] += m.y * p.inv_scale;
-                s[4 * g + 2] += m.z * p.inv_scale;
-                s[4 * g + 3] += m.w * p.inv_scale;
+                float s0 = s[4 * g + 0], s1 = s[4 * g + 1], s2 = s[4 * g + 2], s3 = s[4 * g + 3];
+                mslab.add(mraw[g], p.inv_scale, s0, s1, s2, s3);
+                s[4 * g + 0] = s0, s[4 * g + 1] = s1, s[4 * g + 2] = s2, s[4 * g + 3] = s3;
             }
             next_tile();
         }
@@ -276,7 +275,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_kernel(const PrefillParams
     }
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
+template <int D, bool CAUSAL, int MASKED, bool PAD>
 static int launch_prefill_f32(const PrefillParams& prm, hipStream_t stream) {
     constexpr int BM = 4 * 32;
     PrefillParams p = prm;
@@ -306,7 +305,7 @@ __device__ __forceinline__ void wait_vm_n() {
 //
 // Each wave loads its own tiles into its own LDS buffers, so the loop has no barrier.  The buffers are
 // single: K(t+4) lands while PV(t) runs and V(t+4) while S(t+4) runs (1,024 to 4,096 MFMA cycles each).
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
+template <int D, bool CAUSAL, int MASKED, bool PAD>
 __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(const PrefillParams p) {
     constexpr int NW = 4;
     constexpr int BN = 32;           // keys per tile
@@ -360,9 +359,10 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(co
         }
     };
 
-    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
-    const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
-    const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(q0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
+    const auto mslab = [&] {
+        if constexpr (MASKED != kMaskNone) return MaskSlab<MASKED>(p, b, hq, q0 + l32);
+        else return 0;
+    }();
 
     float qf[HD];
     f32x16 oacc[DT];
@@ -398,10 +398,10 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(co
         const int kbase = t * BN;
         const bool more = t + NW < nt;
         wait_vm_n<INSTR>();  // K(t) landed; V(t), issued after it, may be in flight
-        u32x4 mraw[4];
-        if constexpr (MASKED) {
+        typename MaskSlab<MASKED>::Group mraw[4];
+        if constexpr (MASKED != kMaskNone) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) mraw[g] = buf_ld16(mrs, mrow_off + (uint32_t)((kbase + 8 * g + 4 * hf) * 4));
+            for (int g = 0; g < 4; ++g) mraw[g] = mslab.load(kbase + 8 * g + 4 * hf);
         }
         f32x16 s;
 #pragma unroll
@@ -428,14 +428,12 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(co
         // every K(t) read has returned: K(t+4) may land
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (more) dma(Kt, kp, krow, p.ks_s, t + NW, p.qk_ch);
-        if constexpr (MASKED) {
+        if constexpr (MASKED != kMaskNone) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const f32x4 m = __builtin_bit_cast(f32x4, mraw[g]);
-                s[4 * g + 0] += m.x * p.inv_scale;
-                s[4 * g + 1] += m.y * p.inv_scale;
-                s[4 * g + 2] += m.z * p.inv_scale;
-                s[4 * g + 3] += m.w * p.inv_scale;
+                float s0 = s[4 * g + 0], s1 = s[4 * g + 1], s2 = s[4 * g + 2], s3 = s[4 * g + 3];
+                mslab.add(mraw[g], p.inv_scale, s0, s1, s2, s3);
+                s[4 * g + 0] = s0, s[4 * g + 1] = s1, s[4 * g + 2] = s2, s[4 * g + 3] = s3;
             }
         }
         const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && (kbase + BN - 1 > q0 + p.delta));
@@ -548,7 +546,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(co
     }
 }
 
-template <int D, bool CAUSAL, bool MASKED, bool PAD>
+template <int D, bool CAUSAL, int MASKED, bool PAD>
 static int launch_prefill_f32_ks(const PrefillParams& prm, hipStream_t stream) {
     PrefillParams p = prm;
     p.n_qblocks = (p.Sq + 31) / 32;
@@ -645,7 +643,7 @@ __global__ void __launch_bounds__(256, 1) prefill_f32_wide_kernel(const PrefillP
     };
     static_assert(DCH >= 64, "one 1 KB load instruction covers at most one row");
 
-    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
+    const float* mbase_p = MASKED ? reinterpret_cast<const float*>(p.mask) + b * p.ms_b + hq * p.ms_h : nullptr;
     const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
     const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(q0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
 
@@ -878,7 +876,7 @@ static bool f32_key_split(const PrefillParams& p, int D, bool causal, hipStream_
     return e * cost(sum_ks, longest_ks, heads * (((int64_t)p.Sq + 31) / 32)) < cost(sum, longest, heads * blocks);
 }
 
-template <bool MASKED, bool PAD>
+template <int MASKED, bool PAD>
 static int dispatch_prefill_f32_m(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
     if (f32_key_split(p, D, causal, stream)) {
         if (D == 128)
@@ -893,23 +891,32 @@ static int dispatch_prefill_f32_m(const PrefillParams& p, int D, bool causal, hi
     if (D == 64)
         return causal ? launch_prefill_f32<64, true, MASKED, PAD>(p, stream)
                       : launch_prefill_f32<64, false, MASKED, PAD>(p, stream);
-    if (D == 256)
-        return causal ? launch_prefill_f32_wide<256, true, MASKED, PAD>(p, stream)
-                      : launch_prefill_f32_wide<256, false, MASKED, PAD>(p, stream);
-    if (D == 512)
-        return causal ? launch_prefill_f32_wide<512, true, MASKED, PAD>(p, stream)
-                      : launch_prefill_f32_wide<512, false, MASKED, PAD>(p, stream);
+    if constexpr (MASKED == kMaskNone || MASKED == kMaskF32) {  // wide heads take fp32 masks only
+        if (D == 256)
+            return causal ? launch_prefill_f32_wide<256, true, MASKED, PAD>(p, stream)
+                          : launch_prefill_f32_wide<256, false, MASKED, PAD>(p, stream);
+        if (D == 512)
+            return causal ? launch_prefill_f32_wide<512, true, MASKED, PAD>(p, stream)
+                          : launch_prefill_f32_wide<512, false, MASKED, PAD>(p, stream);
+    }
     return fail(DTATTN_ERR_UNSUPPORTED, "prefill: fp32 kernel head dim %d not supported (64, 128, 256 or 512)", D);
 }
 
 // Entry from dtattn_prefill_fwd once the arguments are validated and `p` is filled.  D is the kernel's
 // head dim (64, 128, 256 or 512); pad: the real head dims (p.qk_ch, p.v_ch chunks of 4 floats) are below it.
 int prefill_f32(const PrefillParams& p, int D, bool causal, bool pad, hipStream_t stream) {
-    if (pad)
-        return p.mask != nullptr ? dispatch_prefill_f32_m<true, true>(p, D, causal, stream)
-                                 : dispatch_prefill_f32_m<false, true>(p, D, causal, stream);
-    return p.mask != nullptr ? dispatch_prefill_f32_m<true, false>(p, D, causal, stream)
-                             : dispatch_prefill_f32_m<false, false>(p, D, causal, stream);
+    const MaskMode mode = mask_mode(p);
+    auto run = [&](auto pad_c) {
+        constexpr bool PAD = decltype(pad_c)::value;
+        switch (mode) {
+            case kMaskF32: return dispatch_prefill_f32_m<kMaskF32, PAD>(p, D, causal, stream);
+            case kMaskBool: return dispatch_prefill_f32_m<kMaskBool, PAD>(p, D, causal, stream);
+            case kMaskBf16: return dispatch_prefill_f32_m<kMaskBf16, PAD>(p, D, causal, stream);
+            case kMaskF16: return dispatch_prefill_f32_m<kMaskF16, PAD>(p, D, causal, stream);
+            default: return dispatch_prefill_f32_m<kMaskNone, PAD>(p, D, causal, stream);
+        }
+    };
+    return pad ? run(std::true_type{}) : run(std::false_type{});
 }
 
 }  // namespace dtattn

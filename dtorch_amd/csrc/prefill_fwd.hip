@@ -28,6 +28,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "dtattn_common.hpp"
 #include "prefill_params.hpp"
 
@@ -44,7 +46,7 @@ __device__ __forceinline__ int kswz(int r) {
 
 // PAD: the real head dims are below D (any multiple of 8, Dv may differ from D); Q/K chunks past
 // p.qk_ch and V chunks past p.v_ch load as zeros, and O chunks past p.v_ch are not stored.
-template <typename T, int D, int QT, bool CAUSAL, bool MASKED, bool PAD>
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD>
 __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams p) {
     constexpr int NW = 4;
     constexpr int BN = 64;
@@ -76,6 +78,8 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
 
     const BlockCoord bc = block_coord<CAUSAL>(p);
     const int qb = bc.qb, b = bc.b, hq = bc.hq, hk = bc.hk;
+    if constexpr (MASKED == kMaskF32)
+        if (p.spans != nullptr && p.spans[b].y >= 0) return;  // run as a key span (prefill_rows64.hip)
 
     const T* qp = reinterpret_cast<const T*>(p.q) + b * p.qs_b + hq * p.qs_h;
     const T* kp = reinterpret_cast<const T*>(p.k) + b * p.ks_b + hk * p.ks_h;
@@ -132,12 +136,12 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
     const int tr_d = 16 * (blk & 1) + 4 * (bl & 3);  // D0 offset within the 32-d tile + 4a
     const int tr_k4 = 4 * (blk >> 1);           // 4 * hf
 
-    // MASKED: the mask slab of (b, hq) behind a buffer resource, so reads past its last row return 0
-    // (those keys are hidden by the ragged-tail mask anyway).  Lane (l32, hf) reads, for query row
-    // wq0 + l32, the four consecutive keys of each of its 4 groups per 32-key tile.
-    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
-    const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
-    const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(wq0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
+    // MASKED: lane (l32, hf) reads, for query row wq0 + l32, the four consecutive keys of each of its 4 groups per
+    // 32-key tile.
+    const auto mslab = [&] {
+        if constexpr (MASKED != kMaskNone) return MaskSlab<MASKED>(p, b, hq, wq0 + l32);
+        else return 0;
+    }();
 
     // One key tile.  Kc/Vc hold tile t; Kn/Vn receive tile t+1.
     auto tile = [&](const T* Kc, const T* Vc, T* Kn, T* Vn, int t) {
@@ -153,7 +157,7 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
         // S block in the non-causal one (measured +2.5% at 256-512 keys, neutral on long rows; the causal
         // kernel would spill); masked kernels after the mask add (the compiler's wait for the mask values
         // would otherwise also wait for the tile loads).
-        constexpr bool kLateLoads = MASKED || !CAUSAL;
+        constexpr bool kLateLoads = MASKED != kMaskNone || !CAUSAL;
         if constexpr (!kLateLoads) next_tile();
         const int kbase = t * BN;
         if (CAUSAL && kbase > wq0 + 31 + p.delta) {  // every row of this wave precedes the tile
@@ -161,11 +165,11 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
             return;
         }
         const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && (kbase + BN - 1 > wq0 + p.delta));
-        u32x4 mraw[KT * 4];
-        if constexpr (MASKED) {
+        typename MaskSlab<MASKED>::Group mraw[MASKED != kMaskNone ? KT * 4 : 1];
+        if constexpr (MASKED != kMaskNone) {
 #pragma unroll
             for (int g = 0; g < KT * 4; ++g)  // keys kbase + 32*(g/4) + 8*(g%4) + 4*hf .. +3
-                mraw[g] = buf_ld16(mrs, mrow_off + (uint32_t)((kbase + 32 * (g >> 2) + 8 * (g & 3) + 4 * hf) * 4));
+                mraw[g] = mslab.load(kbase + 32 * (g >> 2) + 8 * (g & 3) + 4 * hf);
         }
 
         f32x16 s[KT];
@@ -192,14 +196,25 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        if constexpr (MASKED) {
+        // A tile whose keys a bool mask keeps for every row of the wave needs no adds (s + 0): most tiles of a
+        // padding mask.
+        bool add_mask = MASKED != kMaskNone;
+        if constexpr (MASKED == kMaskBool) {
+            uint32_t all = mslab.bytes(mraw[0]);
 #pragma unroll
-            for (int g = 0; g < KT * 4; ++g) {
-                const f32x4 m = __builtin_bit_cast(f32x4, mraw[g]);
-                s[g >> 2][4 * (g & 3) + 0] += m.x * p.inv_scale;
-                s[g >> 2][4 * (g & 3) + 1] += m.y * p.inv_scale;
-                s[g >> 2][4 * (g & 3) + 2] += m.z * p.inv_scale;
-                s[g >> 2][4 * (g & 3) + 3] += m.w * p.inv_scale;
+            for (int g = 1; g < KT * 4; ++g) all &= mslab.bytes(mraw[g]);
+            add_mask = !__all(all == 0x01010101u);
+        }
+        if (add_mask) {
+            if constexpr (MASKED != kMaskNone) {
+#pragma unroll
+                for (int g = 0; g < KT * 4; ++g) {
+                    float s0 = s[g >> 2][4 * (g & 3) + 0], s1 = s[g >> 2][4 * (g & 3) + 1];
+                    float s2 = s[g >> 2][4 * (g & 3) + 2], s3 = s[g >> 2][4 * (g & 3) + 3];
+                    mslab.add(mraw[g], p.inv_scale, s0, s1, s2, s3);
+                    s[g >> 2][4 * (g & 3) + 0] = s0, s[g >> 2][4 * (g & 3) + 1] = s1;
+                    s[g >> 2][4 * (g & 3) + 2] = s2, s[g >> 2][4 * (g & 3) + 3] = s3;
+                }
             }
         }
         if constexpr (kLateLoads) next_tile();
@@ -363,7 +378,7 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
 
 // ------------------------------------------------------------------------------------------------
 
-template <typename T, int D, int QT, bool CAUSAL, bool MASKED, bool PAD>
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD>
 static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     constexpr int BM = 4 * QT * 32;
     PrefillParams p = prm;
@@ -375,7 +390,7 @@ static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     return check_launch("prefill_fwd_kernel");
 }
 
-template <typename T, bool MASKED, bool PAD>
+template <typename T, int MASKED, bool PAD>
 static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
     if (D == 128) {
         return causal ? launch_prefill<T, 128, 1, true, MASKED, PAD>(p, stream)
@@ -390,21 +405,107 @@ static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, hipStr
 
 int prefill_rows64(const PrefillParams& p, bool causal, bool f16, void* ws, size_t ws_bytes, hipStream_t stream);
 bool prefill_rows64_fits(const PrefillParams& p);
+int prefill_rows64_spans(const PrefillParams& p, bool causal, bool f16, hipStream_t stream);
 size_t rows64_sk_workspace(const dtattn_prefill_args* a, int device);
+
+// Kernel head dim of a bf16/fp16 call: the smallest of 64, 128, 256, 512 holding both real head dims.
+static int kernel_head_dim(int64_t D, int64_t Dv) {
+    const int64_t dmax = D > Dv ? D : Dv;
+    return dmax <= 64 ? 64 : dmax <= 128 ? 128 : dmax <= 256 ? 256 : dmax <= 512 ? 512 : 0;
+}
+
+// A mask that is one row of keys per (batch, or batch and head), read once: the row in fp32 at rows + slab * pitch
+// (0 and -inf for a bool mask), which the attention kernels then read for every query without decoding it
+// again, and its key span (PrefillParams::spans).  One workgroup per slab; the row is a few KB, so this is one
+// short launch (about 3 us) ahead of a call of 40 us or more.
+__global__ void __launch_bounds__(256) mask_rows_kernel(const void* mask, int kind, int64_t ms_b, int64_t ms_h, int heads,
+                                                        int Sk, float inv_scale, float* rows, int64_t pitch, int2* spans) {
+    __shared__ int red[4][4];
+    const int slab = blockIdx.x;
+    const int64_t off = (slab / heads) * ms_b + (slab % heads) * ms_h;
+    float* row = rows + slab * pitch;
+    int first = Sk, last = -1, count = 0, other = 0;
+    for (int j = threadIdx.x; j < Sk; j += 256) {
+        float m;
+        if (kind == DTATTN_BOOL) m = reinterpret_cast<const uint8_t*>(mask)[off + j] != 0 ? 0.f : kNegInf;
+        else if (kind == DTATTN_BF16) m = (float)reinterpret_cast<const bf16_t*>(mask)[off + j];
+        else if (kind == DTATTN_FP16) m = (float)reinterpret_cast<const f16_t*>(mask)[off + j];
+        else m = reinterpret_cast<const float*>(mask)[off + j];
+        row[j] = m;
+        if (m * inv_scale != kNegInf) {  // not hidden
+            first = min(first, j);
+            last = max(last, j);
+            ++count;
+            other |= m != 0.f;  // NaN too
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        first = min(first, __shfl_xor(first, d, 64));
+        last = max(last, __shfl_xor(last, d, 64));
+        count += __shfl_xor(count, d, 64);
+        other |= __shfl_xor(other, d, 64);
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) red[0][w] = first, red[1][w] = last, red[2][w] = count, red[3][w] = other;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int i = 1; i < 4; ++i) {
+        first = min(first, red[0][i]);
+        last = max(last, red[1][i]);
+        count += red[2][i];
+        other |= red[3][i];
+    }
+    spans[slab] = count == 0 ? make_int2(0, 0) : other == 0 && count == last + 1 - first ? make_int2(first, last + 1) : make_int2(0, -1);
+}
+
+// Whether mask_rows_kernel runs ahead of a masked call, and the workspace it needs: bf16 / fp16 calls at kernel head
+// dims 64 and 128 whose mask is the same for every query, once they hold 2.4e10 operations (40 us and up at the
+// masked kernels' rate).  Below that its launch costs more than decoding the mask in the attention kernel.
+static size_t mask_rows_workspace(const dtattn_prefill_args* a, const dtattn_mask* mk, int64_t* pitch, int64_t* slabs) {
+    if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16) return 0;
+    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 1 || a->Sk <= 0 || mk->stride[2] != 0) return 0;
+    const int Dk = kernel_head_dim(a->D, a->Dv);
+    if (Dk != 64 && Dk != 128) return 0;
+    const double pairs = (double)a->B * (double)a->Hq * (double)a->Sq * (double)a->Sk * (a->causal != 0 ? 0.5 : 1.0);
+    if (4.0 * Dk * pairs < 2.4e10) return 0;
+    *slabs = a->B * (mk->stride[1] == 0 ? 1 : a->Hq);
+    *pitch = (a->Sk + 3) / 4 * 4;
+    if (*slabs > 0x7fffffff) return 0;
+    return (((size_t)*slabs * sizeof(int2) + 255) & ~(size_t)255) + (size_t)*slabs * *pitch * sizeof(float);
+}
 
 // D is the kernel's head dim (64 or 128); pad: the real head dims are below it.  Head dim 128 without mask or
 // padding runs the 64-rows-per-wave kernel (prefill_rows64.hip), which returns the same bits as
 // prefill_fwd_kernel at 4-9% (non-causal) and 4-14% (causal) more throughput.
 template <typename T>
-static int dispatch_prefill(const PrefillParams& p, int D, bool causal, bool pad, void* ws, size_t ws_bytes,
-                            hipStream_t stream) {
+static int dispatch_prefill(PrefillParams p, int D, bool causal, bool pad, void* ws, size_t ws_bytes, hipStream_t stream) {
+    // Row masks with key spans: the batches that have one run as shorter calls without a mask, on the faster kernel
+    // and without the hidden tiles; prefill_fwd_kernel then runs the others and leaves at once for these (about 4 us
+    // of a call).  4x32/8x2000, left padding up to half: causal 219 -> 103 us, not causal 264 -> 186 us; a mask with
+    // holes 219 -> 222 us.
+    if (p.spans != nullptr) {
+        if (D == 128 && !pad && p.ms_h == 0 && prefill_rows64_fits(p)) {
+            const int st = prefill_rows64_spans(p, causal, __is_same(T, f16_t), stream);
+            if (st != DTATTN_OK) return st;
+        } else {
+            p.spans = nullptr;
+        }
+    }
     if (D == 128 && !pad && p.mask == nullptr && prefill_rows64_fits(p))
         return prefill_rows64(p, causal, __is_same(T, f16_t), ws, ws_bytes, stream);
-    if (pad)
-        return p.mask != nullptr ? dispatch_prefill_m<T, true, true>(p, D, causal, stream)
-                                 : dispatch_prefill_m<T, false, true>(p, D, causal, stream);
-    return p.mask != nullptr ? dispatch_prefill_m<T, true, false>(p, D, causal, stream)
-                             : dispatch_prefill_m<T, false, false>(p, D, causal, stream);
+    const MaskMode mode = mask_mode(p);
+    auto run = [&](auto pad_c) {
+        constexpr bool PAD = decltype(pad_c)::value;
+        switch (mode) {
+            case kMaskF32: return dispatch_prefill_m<T, kMaskF32, PAD>(p, D, causal, stream);
+            case kMaskBool: return dispatch_prefill_m<T, kMaskBool, PAD>(p, D, causal, stream);
+            case kMaskBf16: return dispatch_prefill_m<T, kMaskBf16, PAD>(p, D, causal, stream);
+            case kMaskF16: return dispatch_prefill_m<T, kMaskF16, PAD>(p, D, causal, stream);
+            default: return dispatch_prefill_m<T, kMaskNone, PAD>(p, D, causal, stream);
+        }
+    };
+    return pad ? run(std::true_type{}) : run(std::false_type{});
 }
 
 int prefill_fp8(const dtattn_prefill_args* a, float c, int32_t delta, uint32_t q_and, uint32_t q_xor,
@@ -413,12 +514,6 @@ size_t prefill_fp8_workspace_size(const dtattn_prefill_args* a, int device);
 int prefill_f32(const PrefillParams& p, int D, bool causal, bool pad, hipStream_t stream);
 int prefill_wide(const PrefillParams& p, int D, bool causal, bool bf16, bool pad, hipStream_t stream);
 int wide_key_splits(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, int D, int cu_count);
-
-// Kernel head dim of a bf16/fp16 call: the smallest of 64, 128, 256, 512 holding both real head dims.
-static int kernel_head_dim(int64_t D, int64_t Dv) {
-    const int64_t dmax = D > Dv ? D : Dv;
-    return dmax <= 64 ? 64 : dmax <= 128 ? 128 : dmax <= 256 ? 256 : dmax <= 512 ? 512 : 0;
-}
 
 // Key blocks of a wide-head call on `device` (1: unsplit) and the workspace their partials need:
 // O parts [splits][B][Hq][Sq][Dv] in the input dtype, then (256-byte aligned) LSE parts
@@ -445,13 +540,18 @@ static int stream_device(hipStream_t stream, int* dev) {
                                                                                                : DTATTN_ERR_DEVICE;
 }
 
+static int mask_element_size(int32_t dtype) {
+    return dtype == DTATTN_BOOL ? 1 : dtype == DTATTN_BF16 || dtype == DTATTN_FP16 ? 2 : dtype == DTATTN_FP32 ? 4 : 0;
+}
+
 static bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
 }  // namespace dtattn
 
 using namespace dtattn;
 
-extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream_) {
+// dtattn_prefill_fwd with the mask either in `a` (fp32) or in `mk`, as the caller holds it.
+static int prefill_entry(const dtattn_prefill_args* a, const dtattn_mask* mk, void* stream_) {
     if (a == nullptr) return fail(DTATTN_ERR_INVALID_ARGUMENT, "prefill: args is NULL");
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (a->B < 0 || a->Hq <= 0 || a->Hkv <= 0 || a->Sq < 0 || a->Sk < 0)
@@ -510,6 +610,24 @@ extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream_) {
     if (delta64 < -lim) delta64 = -lim;
     const int32_t delta = (int32_t)delta64;
 
+    if (mk != nullptr) {
+        if (a->mask != nullptr) return fail(DTATTN_ERR_INVALID_ARGUMENT, "prefill: two masks");
+        const int esz = mask_element_size(mk->dtype);
+        if (esz == 0)
+            return fail(DTATTN_ERR_UNSUPPORTED, "prefill: mask dtype %d not supported (bool, bf16, fp16, fp32)", mk->dtype);
+        if (a->dtype == DTATTN_FP8_E4M3FN)
+            return fail(DTATTN_ERR_UNSUPPORTED, "prefill: an attention mask is not supported with fp8 inputs");
+        if (kernel_head_dim(a->D, a->Dv) > 128)
+            return fail(DTATTN_ERR_UNSUPPORTED, "prefill: a mask as stored needs head dims up to 128 (D=%lld, Dv=%lld)",
+                        (long long)a->D, (long long)a->Dv);
+        for (int j = 0; j < 3; ++j)
+            if (mk->stride[j] < 0)
+                return fail(DTATTN_ERR_UNSUPPORTED, "prefill: mask stride[%d]=%lld is negative", j, (long long)mk->stride[j]);
+        if (mk->data == nullptr || reinterpret_cast<uintptr_t>(mk->data) % (uintptr_t)esz != 0)
+            return fail(DTATTN_ERR_INVALID_ARGUMENT, "prefill: mask pointer is null or not aligned to its elements");
+        if (((a->Sq - 1) * mk->stride[2] + a->Sk + 64) * esz + 64 >= ((int64_t)1 << 32))
+            return fail(DTATTN_ERR_UNSUPPORTED, "prefill: mask slab of one (batch, head) exceeds 4 GB");
+    }
     if (a->mask != nullptr) {
         if (a->dtype == DTATTN_FP8_E4M3FN)
             return fail(DTATTN_ERR_UNSUPPORTED, "prefill: an attention mask is not supported with fp8 inputs");
@@ -557,8 +675,11 @@ extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream_) {
     p.delta = delta;
     p.c = c;
     p.xcd_map = (p.B * p.Hkv) % 8 == 0 ? 1 : 0;
-    p.mask = a->mask;
-    p.ms_b = a->mask_stride[0], p.ms_h = a->mask_stride[1], p.ms_l = a->mask_stride[2];
+    p.mask = mk != nullptr ? mk->data : a->mask;
+    const int64_t* ms = mk != nullptr ? mk->stride : a->mask_stride;
+    p.ms_b = ms[0], p.ms_h = ms[1], p.ms_l = ms[2];
+    p.mask_kind = mk != nullptr ? mk->dtype : DTATTN_FP32;
+    p.spans = nullptr;
     p.inv_scale = 1.0f / scale;
     p.nsplit = 1;
     p.kblock = (int32_t)(a->Sk > 0 ? a->Sk : 1);
@@ -567,6 +688,23 @@ extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream_) {
     p.q_and = sp.q_and;
     p.q_xor = sp.q_xor;
     const bool causal = a->causal != 0;
+    if (mk != nullptr && a->workspace != nullptr && (reinterpret_cast<uintptr_t>(a->workspace) & 255u) == 0) {
+        int64_t pitch = 0, slabs = 0;
+        const size_t need = mask_rows_workspace(a, mk, &pitch, &slabs);
+        if (need > 0 && need <= a->workspace_bytes) {
+            const int heads = (int)(slabs / a->B);
+            int2* spans = reinterpret_cast<int2*>(a->workspace);
+            float* rows = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + (((size_t)slabs * sizeof(int2) + 255) & ~(size_t)255));
+            hipLaunchKernelGGL(mask_rows_kernel, dim3((unsigned)slabs), dim3(256), 0, stream, mk->data, mk->dtype, mk->stride[0],
+                               mk->stride[1], heads, p.Sk, p.inv_scale, rows, pitch, spans);
+            const int st = check_launch("mask_rows_kernel");
+            if (st != DTATTN_OK) return st;
+            p.mask = rows;
+            p.mask_kind = DTATTN_FP32;
+            p.ms_b = heads * pitch, p.ms_h = heads > 1 ? pitch : 0, p.ms_l = 0;
+            p.spans = spans;
+        }
+    }
     if (a->dtype == DTATTN_FP32) {
         // kernel head dim 64, 128, 256 or 512 (the last two on the wide fp32 kernel); smaller real dims
         // (multiples of 4, D and Dv independent) are padded
@@ -627,6 +765,18 @@ extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream_) {
     }
     if (a->dtype == DTATTN_BF16) return dispatch_prefill<bf16_t>(p, Dk, causal, pad, a->workspace, a->workspace_bytes, stream);
     return dispatch_prefill<f16_t>(p, Dk, causal, pad, a->workspace, a->workspace_bytes, stream);
+}
+
+extern "C" int dtattn_prefill_fwd(const dtattn_prefill_args* a, void* stream) { return prefill_entry(a, nullptr, stream); }
+
+extern "C" int dtattn_prefill_masked(const dtattn_prefill_args* a, const dtattn_mask* mask, void* stream) {
+    return prefill_entry(a, mask, stream);
+}
+
+extern "C" size_t dtattn_prefill_masked_workspace_size(const dtattn_prefill_args* a, const dtattn_mask* mask) {
+    if (a == nullptr || mask == nullptr) return 0;
+    int64_t pitch = 0, slabs = 0;
+    return mask_rows_workspace(a, mask, &pitch, &slabs);
 }
 
 extern "C" size_t dtattn_prefill_workspace_size(const dtattn_prefill_args* a) {

@@ -51,7 +51,9 @@ struct DmaOffsets<2> {
 
 }  // namespace
 
-template <typename T, bool CAUSAL, int NW>
+// SPAN: batch b attends to keys [p.spans[b].x, p.spans[b].y) only, i.e. it is the call on K and V from the first
+// of them, with that many keys and the causal diagonal moved along; batches without a span are left alone.
+template <typename T, bool CAUSAL, int NW, bool SPAN>
 __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const PrefillParams p) {
     typedef typename Elem<T>::vec4 V4;
     constexpr int D = 128, BN = 64, BM = NW * 64, DCH = 16, INSTR = 16 / NW;
@@ -69,18 +71,27 @@ __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const Prefil
     const T* qp = reinterpret_cast<const T*>(p.q) + b * p.qs_b + hq * p.qs_h;
     const T* kp = reinterpret_cast<const T*>(p.k) + b * p.ks_b + hk * p.ks_h;
     const T* vp = reinterpret_cast<const T*>(p.v) + b * p.vs_b + hk * p.vs_h;
+    int sk = p.Sk, delta = p.delta;
+    if constexpr (SPAN) {
+        const int2 sp = p.spans[b];
+        if (sp.y < 0) return;
+        sk = __builtin_amdgcn_readfirstlane(sp.y - sp.x);
+        delta -= sp.x;
+        kp += sp.x * p.ks_s;
+        vp += sp.x * p.vs_s;
+    }
 
     const int q0 = bc.qb * BM;
     const int wq0 = q0 + wave * 64;
-    int kend = p.Sk;
+    int kend = sk;
     if (CAUSAL) {
-        const int lim = q0 + BM + p.delta;  // keys < lim can be visible to the workgroup
-        kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
+        const int lim = q0 + BM + delta;  // keys < lim can be visible to the workgroup
+        kend = lim < 0 ? 0 : (lim < sk ? lim : sk);
     }
     const int nt = (kend + BN - 1) / BN;
     int tw = nt;  // tiles this wave computes; the others it only loads and waits through
     if (CAUSAL) {
-        const int last = wq0 + 63 + p.delta;
+        const int last = wq0 + 63 + delta;
         tw = last < 0 ? 0 : min(nt, last / BN + 1);
     }
     tw = __builtin_amdgcn_readfirstlane(tw);
@@ -100,7 +111,7 @@ __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const Prefil
         doff[INSTR + i] = (uint32_t)(r * vrow + cc * 16);
     }
     auto dma = [&](int buf, const T* base, int pitch, int64_t stride, int t, int first) {
-        const int rows = min(BN, p.Sk - t * BN);
+        const int rows = min(BN, sk - t * BN);
         const uint32_t nbytes = (uint32_t)((rows - 1) * pitch + D * (int)sizeof(T));
         const auto rs = make_rsrc(base + (int64_t)t * BN * stride, nbytes);
         T* dst = smem + buf * BN * D;
@@ -129,8 +140,8 @@ __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const Prefil
     u32x2 lim;
 #pragma unroll
     for (int X = 0; X < 2; ++X) {
-        int v = p.Sk - 1;
-        if (CAUSAL) v = min(v, wq0 + 32 * X + l32 + p.delta);
+        int v = sk - 1;
+        if (CAUSAL) v = min(v, wq0 + 32 * X + l32 + delta);
         lim[X] = (uint32_t)(v - 4 * hf);
     }
 
@@ -164,7 +175,7 @@ __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const Prefil
     for (int i = 0; i < 32; ++i) OA01[i] = 0.f, OA23[i] = 0.f, OB01[i] = 0.f, OB23[i] = 0.f;
     float mA = kNegInf, mB = kNegInf, lA = 0.f, lB = 0.f;
     const float c = p.c;
-    const int kd = wq0 + p.delta;
+    const int kd = wq0 + delta;
     const uint64_t kb64 = (uint64_t)(uintptr_t)kp, vb64 = (uint64_t)(uintptr_t)vp;
     const uint32_t klo = (uint32_t)kb64, khi = (uint32_t)(kb64 >> 32);
     const uint32_t vlo = (uint32_t)vb64, vhi = (uint32_t)(vb64 >> 32);
@@ -179,7 +190,7 @@ __global__ void __launch_bounds__(64 * NW, 1) prefill_rows64_kernel(const Prefil
     : "+{a[0:31]}"(OA01), "+{a[32:63]}"(OA23), "+{a[64:95]}"(OB01), "+{a[96:127]}"(OB23), [mA] "+v"(mA),       \
       [mB] "+v"(mB), [lA] "+v"(lA), [lB] "+v"(lB)                                                                \
     : "{a[128:159]}"(QA), "{a[160:191]}"(QB), "{v[200:215]}"(addr), [nt] "s"(nt), [tw] "s"(tw), [c] "s"(c),    \
-      [sk] "s"(p.Sk), [kd] "s"(kd), [kp] "s"(krow), [vp] "s"(vrow), [klo] "s"(klo), [khi] "s"(khi),            \
+      [sk] "s"(sk), [kd] "s"(kd), [kp] "s"(krow), [vp] "s"(vrow), [klo] "s"(klo), [khi] "s"(khi),            \
       [vlo] "s"(vlo), [vhi] "s"(vhi), [m0base] "s"(m0base)
 #define DTATTN_ROWS64_RUN(PROG)                                                                                \
     if constexpr (NW == 4)                                                                                     \
@@ -259,7 +270,7 @@ __device__ __forceinline__ int gqa_item(int w, int k, int G, int xcd_map) {
     return (k & 1) ? (k + 1) * G - 1 - w : k * G + w;
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool SPAN>
 __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const PrefillParams p, int n_items) {
     typedef typename Elem<T>::vec4 V4;
     constexpr int D = 128, BN = 64, DCH = 16, INSTR = 4;
@@ -289,6 +300,7 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
 
     struct Item {
         int b, hq, q0, nt;
+        int sk, delta;  // keys and causal offset: SPAN's (sk < 0: the batch has none), else the call's
         const T *qp, *kp, *vp;
     };
     auto item_at = [&](int bid) {
@@ -297,19 +309,28 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
         it.b = bc.b;
         it.hq = bc.hk * p.group + (bc.hq - bc.hk * nsub) * 4 + wave;
         it.q0 = bc.qb * 64;
-        int kend = p.Sk;
+        it.sk = p.Sk, it.delta = p.delta;
+        int first = 0;
+        if constexpr (SPAN) {
+            const int2 sp = p.spans[it.b];
+            first = __builtin_amdgcn_readfirstlane(sp.x);
+            it.sk = __builtin_amdgcn_readfirstlane(sp.y) - first;
+            it.delta -= first;
+        }
+        int kend = it.sk;
         if (CAUSAL) {
-            const int lim = it.q0 + 64 + p.delta;
-            kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
+            const int lim = it.q0 + 64 + it.delta;
+            kend = lim < 0 ? 0 : (lim < it.sk ? lim : it.sk);
         }
         it.nt = (kend + BN - 1) / BN;
         it.qp = reinterpret_cast<const T*>(p.q) + it.b * p.qs_b + it.hq * p.qs_h;
         it.kp = reinterpret_cast<const T*>(p.k) + it.b * p.ks_b + bc.hk * p.ks_h;
         it.vp = reinterpret_cast<const T*>(p.v) + it.b * p.vs_b + bc.hk * p.vs_h;
+        if constexpr (SPAN) it.kp += first * p.ks_s, it.vp += first * p.vs_s;
         return it;
     };
-    auto dma = [&](int buf, const T* base, int pitch, int64_t stride, int t, int first) {
-        const int rows = min(BN, p.Sk - t * BN);
+    auto dma = [&](int buf, const T* base, int pitch, int64_t stride, int t, int sk, int first) {
+        const int rows = min(BN, sk - t * BN);
         const uint32_t nbytes = (uint32_t)((rows - 1) * pitch + D * (int)sizeof(T));
         const auto rs = make_rsrc(base + (int64_t)t * BN * stride, nbytes);
         T* dst = smem + buf * BN * D;
@@ -319,9 +340,9 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
     u32x32 QA, QB;
     auto prefetch = [&](const Item& it) {
         if (it.nt > 0) {
-            dma(0, it.kp, krow, p.ks_s, 0, 0);
-            dma(2, it.vp, vrow, p.vs_s, 0, INSTR);
-            if (it.nt > 1) dma(1, it.kp, krow, p.ks_s, 1, 0);
+            dma(0, it.kp, krow, p.ks_s, 0, it.sk, 0);
+            dma(2, it.vp, vrow, p.vs_s, 0, it.sk, INSTR);
+            if (it.nt > 1) dma(1, it.kp, krow, p.ks_s, 1, it.sk, 0);
         }
         const T* qa = it.qp + (int64_t)min(it.q0 + l32, p.Sq - 1) * p.qs_s + hf * 8;
         const T* qb = it.qp + (int64_t)min(it.q0 + 32 + l32, p.Sq - 1) * p.qs_s + hf * 8;
@@ -339,9 +360,19 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
             : "memory");
     };
 
-    if ((int)blockIdx.x >= n_items) return;
+    // The workgroup's next item from its k-th on (advances k), or false: SPAN skips the items of batches without one.
+    auto next_item = [&](int& k, Item& it) {
+        for (;; ++k) {
+            const int bid = gqa_item(blockIdx.x, k, G, p.xcd_map);
+            if (bid >= n_items) return false;
+            it = item_at(bid);
+            if (!SPAN || it.sk >= 0) return true;
+        }
+    };
+
     int k = 0;
-    Item it = item_at(gqa_item(blockIdx.x, 0, G, p.xcd_map));
+    Item it;
+    if (!next_item(k, it)) return;
     prefetch(it);
     while (true) {
         u32x16 addr;
@@ -361,8 +392,8 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
         u32x2 lim;
 #pragma unroll
         for (int X = 0; X < 2; ++X) {
-            int v = p.Sk - 1;
-            if (CAUSAL) v = min(v, it.q0 + 32 * X + l32 + p.delta);
+            int v = it.sk - 1;
+            if (CAUSAL) v = min(v, it.q0 + 32 * X + l32 + it.delta);
             lim[X] = (uint32_t)(v - 4 * hf);
         }
         f32x32 OA01, OA23, OB01, OB23;
@@ -370,7 +401,7 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
         for (int i = 0; i < 32; ++i) OA01[i] = 0.f, OA23[i] = 0.f, OB01[i] = 0.f, OB23[i] = 0.f;
         float mA = kNegInf, mB = kNegInf, lA = 0.f, lB = 0.f;
         const float c = p.c;
-        const int kd = it.q0 + p.delta;
+        const int kd = it.q0 + it.delta, sk = it.sk;
         const int nt = __builtin_amdgcn_readfirstlane(it.nt), tw = nt;
         const uint64_t kb64 = (uint64_t)(uintptr_t)it.kp, vb64 = (uint64_t)(uintptr_t)it.vp;
         const uint32_t klo = __builtin_amdgcn_readfirstlane((uint32_t)kb64);
@@ -386,7 +417,7 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
     : "+{a[0:31]}"(OA01), "+{a[32:63]}"(OA23), "+{a[64:95]}"(OB01), "+{a[96:127]}"(OB23), [mA] "+v"(mA),       \
       [mB] "+v"(mB), [lA] "+v"(lA), [lB] "+v"(lB)                                                                \
     : "{a[128:159]}"(QA), "{a[160:191]}"(QB), "{v[200:215]}"(addr), [nt] "s"(nt), [tw] "s"(tw), [c] "s"(c),    \
-      [sk] "s"(p.Sk), [kd] "s"(kd), [kp] "s"(krow), [vp] "s"(vrow), [klo] "s"(klo), [khi] "s"(khi),            \
+      [sk] "s"(sk), [kd] "s"(kd), [kp] "s"(krow), [vp] "s"(vrow), [klo] "s"(klo), [khi] "s"(khi),            \
       [vlo] "s"(vlo), [vhi] "s"(vhi), [m0base] "s"(m0base), "{v[216:223]}"(doff), "{v[224:225]}"(lim)
             constexpr bool F16 = __is_same(T, f16_t);
             if constexpr (F16 && CAUSAL) asm volatile(DTATTN_ROWS64_PROGRAM_F16_4_1 DTATTN_ROWS64_GQA_OPERANDS : DTATTN_ROWS64_CLOBBERS);
@@ -400,12 +431,8 @@ __global__ void __launch_bounds__(256, 1) prefill_rows64_gqa_kernel(const Prefil
         lds_barrier();
         const Item cur = it;
         ++k;
-        const int nbid = gqa_item(blockIdx.x, k, G, p.xcd_map);
-        const bool more = nbid < n_items;
-        if (more) {
-            it = item_at(nbid);
-            prefetch(it);
-        }
+        const bool more = next_item(k, it);
+        if (more) prefetch(it);
         // Epilogue: normalise, stage O through this wave's 64 rows of LDS (16-byte chunk c of row r at
         // c ^ (r % 16)) for 16-byte coalesced row stores, LSE
         T* Os = ostage + wave * 64 * D;
@@ -788,14 +815,14 @@ __global__ void __launch_bounds__(256) rows64_sk_merge_kernel(const PrefillParam
     }
 }
 
-template <typename T, bool CAUSAL, int NW>
+template <typename T, bool CAUSAL, int NW, bool SPAN>
 static int launch_rows64(const PrefillParams& prm, hipStream_t stream) {
     PrefillParams p = prm;
     p.n_qblocks = (p.Sq + 64 * NW - 1) / (64 * NW);
     const int64_t grid = (int64_t)p.n_qblocks * p.B * p.Hq;
     if (grid == 0) return DTATTN_OK;
     if (grid > 0x7fffffff) return fail(DTATTN_ERR_UNSUPPORTED, "prefill grid too large (%lld blocks)", (long long)grid);
-    hipLaunchKernelGGL((prefill_rows64_kernel<T, CAUSAL, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, stream, p);
+    hipLaunchKernelGGL((prefill_rows64_kernel<T, CAUSAL, NW, SPAN>), dim3((unsigned)grid), dim3(64 * NW), 0, stream, p);
     return check_launch("prefill_rows64_kernel");
 }
 
@@ -811,7 +838,7 @@ static int rows64_stream_device(hipStream_t stream, int* dev) {
                                                                                                : DTATTN_ERR_DEVICE;
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool SPAN>
 static int launch_rows64_gqa(const PrefillParams& prm, int cus, hipStream_t stream) {
     PrefillParams p = prm;
     p.n_qblocks = (p.Sq + 63) / 64;
@@ -820,7 +847,7 @@ static int launch_rows64_gqa(const PrefillParams& prm, int cus, hipStream_t stre
     if (n_items > 0x7fffffff) return fail(DTATTN_ERR_UNSUPPORTED, "prefill: too many work items");
     int grid = n_items < cus ? (int)n_items : cus;
     if (p.xcd_map) grid &= ~7;  // the item map deals items to XCDs in groups of 8 (n_items is a multiple of 8)
-    hipLaunchKernelGGL((prefill_rows64_gqa_kernel<T, CAUSAL>), dim3((unsigned)grid), dim3(256), 0, stream, p,
+    hipLaunchKernelGGL((prefill_rows64_gqa_kernel<T, CAUSAL, SPAN>), dim3((unsigned)grid), dim3(256), 0, stream, p,
                        (int)n_items);
     return check_launch("prefill_rows64_gqa_kernel");
 }
@@ -880,6 +907,17 @@ static int launch_rows64_sk(const PrefillParams& p, const Rows64Sk& sk, hipStrea
     return check_launch("rows64_sk_merge_kernel");
 }
 
+// Grouped-query calls with groups of 4k heads and a positive scale take the persistent form.
+template <typename T, bool CAUSAL, bool SPAN>
+static int launch_rows64_plain(const PrefillParams& p, bool gqa, hipStream_t stream) {
+    int dev = 0;
+    dtattn_device_peaks pk;
+    if (gqa && rows64_stream_device(stream, &dev) == DTATTN_OK && dtattn_get_device_peaks(dev, &pk) == DTATTN_OK &&
+        pk.cu_count >= 8)
+        return launch_rows64_gqa<T, CAUSAL, SPAN>(p, pk.cu_count, stream);
+    return launch_rows64<T, CAUSAL, CAUSAL ? 2 : 4, SPAN>(p, stream);
+}
+
 // ws / ws_bytes: the caller's workspace (may be NULL); non-causal row-layout calls whose grid would leave a
 // ragged last round take the stream-K form when it holds the records.
 int prefill_rows64(const PrefillParams& p, bool causal, bool f16, void* ws, size_t ws_bytes, hipStream_t stream) {
@@ -898,22 +936,19 @@ int prefill_rows64(const PrefillParams& p, bool causal, bool f16, void* ws, size
             return f16 ? launch_rows64_sk<f16_t, false>(p, sk, stream) : launch_rows64_sk<bf16_t, false>(p, sk, stream);
         }
     }
-    // grouped-query calls with groups of 4k heads and a positive scale take the persistent form
-    if (gqa_form && positive) {
-        int dev = 0;
-        dtattn_device_peaks pk;
-        if (rows64_stream_device(stream, &dev) == DTATTN_OK && dtattn_get_device_peaks(dev, &pk) == DTATTN_OK &&
-            pk.cu_count >= 8) {
-            if (f16)
-                return causal ? launch_rows64_gqa<f16_t, true>(p, pk.cu_count, stream)
-                              : launch_rows64_gqa<f16_t, false>(p, pk.cu_count, stream);
-            return causal ? launch_rows64_gqa<bf16_t, true>(p, pk.cu_count, stream)
-                          : launch_rows64_gqa<bf16_t, false>(p, pk.cu_count, stream);
-        }
-    }
-    if (f16)
-        return causal ? launch_rows64<f16_t, true, 2>(p, stream) : launch_rows64<f16_t, false, 4>(p, stream);
-    return causal ? launch_rows64<bf16_t, true, 2>(p, stream) : launch_rows64<bf16_t, false, 4>(p, stream);
+    return f16 ? (causal ? launch_rows64_plain<f16_t, true, false>(p, gqa_form && positive, stream)
+                         : launch_rows64_plain<f16_t, false, false>(p, gqa_form && positive, stream))
+               : (causal ? launch_rows64_plain<bf16_t, true, false>(p, gqa_form && positive, stream)
+                         : launch_rows64_plain<bf16_t, false, false>(p, gqa_form && positive, stream));
+}
+
+// The batches of a row mask that have a key span (p.spans): the same kernels on those keys alone.
+int prefill_rows64_spans(const PrefillParams& p, bool causal, bool f16, hipStream_t stream) {
+    const bool gqa_form = p.group >= 4 && p.group % 4 == 0 && p.q_and == 0xffffffffu && p.q_xor == 0u;
+    return f16 ? (causal ? launch_rows64_plain<f16_t, true, true>(p, gqa_form, stream)
+                         : launch_rows64_plain<f16_t, false, true>(p, gqa_form, stream))
+               : (causal ? launch_rows64_plain<bf16_t, true, true>(p, gqa_form, stream)
+                         : launch_rows64_plain<bf16_t, false, true>(p, gqa_form, stream));
 }
 
 }  // namespace dtattn

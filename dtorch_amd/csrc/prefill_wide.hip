@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(64 * 2 * NRG, 1) prefill_wide_kernel(const Pre
     const int tr_d = 16 * (blk & 1) + 4 * (bl & 3);
     const int tr_k4 = 4 * (blk >> 1);
 
-    const float* mbase_p = MASKED ? p.mask + b * p.ms_b + hq * p.ms_h : nullptr;
+    const float* mbase_p = MASKED ? reinterpret_cast<const float*>(p.mask) + b * p.ms_b + hq * p.ms_h : nullptr;
     const auto mrs = make_rsrc(mbase_p, MASKED ? (uint32_t)((((int64_t)(p.Sq - 1) * p.ms_l + p.Sk) * 4)) : 0u);
     const uint32_t mrow_off = MASKED ? (uint32_t)((int64_t)min(wq0 + l32, p.Sq - 1) * p.ms_l * 4) : 0u;
 

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define DTATTN_ABI_VERSION 10
+#define DTATTN_ABI_VERSION 11
 
 /* Softmax scale fields (ABI version 8): NaN selects 1/sqrt(D) (computed in double and rounded once to
  * float, as libtorch computes its default, from ABI version 10); any finite value is used as given,
@@ -43,7 +43,8 @@ typedef enum {
     DTATTN_BF16 = 0,
     DTATTN_FP16 = 1,
     DTATTN_FP8_E4M3FN = 2, /* OCP e4m3fn, max 448, per-head descales */
-    DTATTN_FP32 = 3
+    DTATTN_FP32 = 3,
+    DTATTN_BOOL = 4 /* attention masks only: one byte, 1 keeps a key, 0 hides it */
 } dtattn_dtype;
 
 /* Prefill / per-block attention: O = softmax(scale * Q K^T [causal]) V, plus the per-row LSE.
@@ -108,6 +109,24 @@ typedef struct {
 } dtattn_prefill_args;
 
 int dtattn_prefill_fwd(const dtattn_prefill_args* args, void* stream);
+
+/* dtattn_prefill_fwd with the attention mask as the caller holds it (ABI version 11; args->mask is NULL):
+ * boolean (a byte of 1 keeps a key, 0 hides it), or added to the logits from bf16, fp16 or fp32.  Element
+ * (b, h, i, j) is data[b*stride[0] + h*stride[1] + i*stride[2] + j] (key stride 1, any strides >= 0, base aligned
+ * to its elements).  Same results as the fp32 form of the same mask, without its conversion pass.  Head dims
+ * up to 128 (D and Dv); BF16/FP16/FP32 inputs. */
+typedef struct {
+    const void* data;
+    int64_t stride[3]; /* B, H, Sq; 0 broadcasts */
+    int32_t dtype;     /* DTATTN_BOOL, DTATTN_BF16, DTATTN_FP16 or DTATTN_FP32 */
+} dtattn_mask;
+
+int dtattn_prefill_masked(const dtattn_prefill_args* args, const dtattn_mask* mask, void* stream);
+/* Workspace bytes (optional, 256-byte aligned) dtattn_prefill_masked can use: a large call whose mask is the same for
+ * every query (a padding mask) first reads the mask once into fp32 rows and finds each batch's span of visible
+ * keys.  Where the mask hides every key outside one span and adds nothing inside it, the keys outside are not read
+ * at all. */
+size_t dtattn_prefill_masked_workspace_size(const dtattn_prefill_args* args, const dtattn_mask* mask);
 /* Workspace bytes dtattn_prefill_fwd can use for `args` on the current device (0 when it would not
  * split the keys); 256-byte aligned pointers expected. */
 size_t dtattn_prefill_workspace_size(const dtattn_prefill_args* args);
