@@ -28,6 +28,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dtattn_common.hpp"
@@ -46,8 +47,10 @@ __device__ __forceinline__ int kswz(int r) {
 
 // PAD: the real head dims are below D (any multiple of 8, Dv may differ from D); Q/K chunks past
 // p.qk_ch and V chunks past p.v_ch load as zeros, and O chunks past p.v_ch are not stored.
-template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD>
-__global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams p) {
+// KG: key groups.  KG * 4 waves share the 128 query rows, group g takes key tiles g, g + KG, ... through its own LDS
+// buffers, and the groups' (O, max, sum) are merged in fp32 through LDS: for grids that leave CUs idle otherwise.
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG = 1>
+__global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel(const PrefillParams p) {
     constexpr int NW = 4;
     constexpr int BN = 64;
     constexpr int BM = NW * 32;
@@ -65,14 +68,19 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
     // K and V tiles, double-buffered, each [64 keys][D] with 16-byte chunk c of row r at c ^ kswz(r).
     // Four distinct LDS objects so the compiler's alias analysis can tell an in-flight load into one
     // buffer from the reads of the others.
-    __shared__ __attribute__((aligned(16))) T Ka[BN * D];
-    __shared__ __attribute__((aligned(16))) T Kb[BN * D];
-    __shared__ __attribute__((aligned(16))) T Va[BN * D];
-    __shared__ __attribute__((aligned(16))) T Vb[BN * D];
+    __shared__ __attribute__((aligned(16))) T Ka_[KG * BN * D];
+    __shared__ __attribute__((aligned(16))) T Kb_[KG * BN * D];
+    __shared__ __attribute__((aligned(16))) T Va_[KG * BN * D];
+    __shared__ __attribute__((aligned(16))) T Vb_[KG * BN * D];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: LDS bases stay scalar
+    const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);  // wave-uniform: LDS bases stay scalar
+    const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+    T* const Ka = Ka_ + kg * BN * D;
+    T* const Kb = Kb_ + kg * BN * D;
+    T* const Va = Va_ + kg * BN * D;
+    T* const Vb = Vb_ + kg * BN * D;
     const int l32 = lane & 31;
     const int hf = lane >> 5;
 
@@ -143,16 +151,17 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
         else return 0;
     }();
 
-    // One key tile.  Kc/Vc hold tile t; Kn/Vn receive tile t+1.
+    // One key tile.  Kc/Vc hold tile t; Kn/Vn receive the group's next tile.
     auto tile = [&](const T* Kc, const T* Vc, T* Kn, T* Vn, int t) {
         wait_vmem();
         lds_barrier();  // tile t landed everywhere; every wave finished tile t-1 (so Kn/Vn are free)
         auto next_tile = [&]() {
-            if (t + 1 < nt) {
-                dma(Kn, kp, krow, p.ks_s, t + 1, p.qk_ch);
-                dma(Vn, vp, vrow, p.vs_s, t + 1, p.v_ch);
+            if (t + KG < nt) {
+                dma(Kn, kp, krow, p.ks_s, t + KG, p.qk_ch);
+                dma(Vn, vp, vrow, p.vs_s, t + KG, p.v_ch);
             }
         };
+        if (KG > 1 && t >= nt) return;  // a group's last round may be short
         // Issue point of the next tile's loads: at the tile start in the causal kernel; after this tile's
         // S block in the non-causal one (measured +2.5% at 256-512 keys, neutral on long rows; the causal
         // kernel would spill); masked kernels after the mask add (the compiler's wait for the mask values
@@ -307,9 +316,9 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
         if constexpr (!CAUSAL) __builtin_amdgcn_s_setprio(0);
     };
 
-    if (nt > 0) {
-        dma(Ka, kp, krow, p.ks_s, 0, p.qk_ch);
-        dma(Va, vp, vrow, p.vs_s, 0, p.v_ch);
+    if (kg < nt) {
+        dma(Ka, kp, krow, p.ks_s, kg, p.qk_ch);
+        dma(Va, vp, vrow, p.vs_s, kg, p.v_ch);
     }
     // Q fragments: lane holds query l32, d = ks*16 + hf*8 .. +8.  Issued after tile 0's loads so that
     // the two share one memory latency.  The loads are unconditional, so they issue back to back (a
@@ -330,14 +339,50 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
     // Q fragments (and tile 0) complete here, visibly to the compiler, so that it inserts no load
     // waits inside the loop (where they would also drain the asynchronous tile loads).
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    for (int t = 0; t < nt; t += 2) {  // unrolled by two so each tile names its buffers statically
-        tile(Ka, Va, Kb, Vb, t);
-        if (t + 1 < nt) tile(Kb, Vb, Ka, Va, t + 1);
+    for (int t = 0; t < nt; t += 2 * KG) {  // unrolled by two so each tile names its buffers statically
+        tile(Ka, Va, Kb, Vb, t + kg);
+        if (t + KG < nt) tile(Kb, Vb, Ka, Va, t + KG + kg);
+    }
+    if constexpr (KG > 1) {
+        // Groups past the first leave their 16 DT accumulators, max and sum per lane in LDS; the first merges them.
+        __syncthreads();
+        auto part = [&](int g) {  // [16 DT][64 lanes] of this wave's rows from group g: KG slots per buffer
+            const int s = (g - 1) * NW + wave;
+            T* const buf = s < KG ? Ka_ : s < 2 * KG ? Kb_ : Va_;
+            return reinterpret_cast<float*>(buf + (s % KG) * BN * D);
+        };
+        float* const ml = reinterpret_cast<float*>(Vb_);
+        if (kg > 0) {
+            float* const dst = part(kg);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) dst[(16 * dt + i) * 64 + lane] = oacc[dt][i];
+            ml[((kg * NW + wave) * 2 + 0) * 64 + lane] = mrow;
+            ml[((kg * NW + wave) * 2 + 1) * 64 + lane] = lrow;
+        }
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int g = 1; g < KG; ++g) {
+                const float* const src = part(g);
+                const float mg = ml[((g * NW + wave) * 2 + 0) * 64 + lane], lg = ml[((g * NW + wave) * 2 + 1) * 64 + lane];
+                const float mm = fmaxf(mrow, mg), mb = mm == kNegInf ? 0.f : mm;  // -inf: no visible key, weight 0
+                const float a0 = fast_exp2(mrow - mb), ag = fast_exp2(mg - mb);
+                mrow = mm;
+                lrow = lrow * a0 + lg * ag;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a0 + src[(16 * dt + i) * 64 + lane] * ag;
+            }
+        }
     }
 
     // Epilogue: normalise, stage O through LDS (wave w in a 32-row slab of Ka/Kb; 16-byte chunk c of
     // row r at c ^ (r % DCH)) for 16-byte coalesced row stores, and write the LSE.
     __syncthreads();
+    if (KG > 1 && kg > 0) return;
     T* Os = (wave < 2 ? Ka : Kb) + (wave & 1) * 32 * D;
     {
         const float l = sum_xor32(lrow);
@@ -378,7 +423,7 @@ __global__ void __launch_bounds__(256, 2) prefill_fwd_kernel(const PrefillParams
 
 // ------------------------------------------------------------------------------------------------
 
-template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD>
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG = 1>
 static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     constexpr int BM = 4 * QT * 32;
     PrefillParams p = prm;
@@ -386,12 +431,20 @@ static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     const int64_t grid = (int64_t)p.n_qblocks * p.B * p.Hq;
     if (grid == 0) return DTATTN_OK;
     if (grid > 0x7fffffff) return fail(DTATTN_ERR_UNSUPPORTED, "prefill grid too large (%lld blocks)", (long long)grid);
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, QT, CAUSAL, MASKED, PAD>), dim3((unsigned)grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, QT, CAUSAL, MASKED, PAD, KG>), dim3((unsigned)grid), dim3(256 * KG), 0, stream, p);
     return check_launch("prefill_fwd_kernel");
 }
 
 template <typename T, int MASKED, bool PAD>
-static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
+static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, int kg, hipStream_t stream) {
+    if constexpr (MASKED == kMaskNone && !PAD) {
+        if (kg > 1 && D == 128)
+            return causal ? launch_prefill<T, 128, 1, true, MASKED, PAD, 2>(p, stream)
+                          : launch_prefill<T, 128, 1, false, MASKED, PAD, 2>(p, stream);
+        if (kg > 1 && D == 64)
+            return causal ? launch_prefill<T, 64, 1, true, MASKED, PAD, 2>(p, stream)
+                          : launch_prefill<T, 64, 1, false, MASKED, PAD, 2>(p, stream);
+    }
     if (D == 128) {
         return causal ? launch_prefill<T, 128, 1, true, MASKED, PAD>(p, stream)
                       : launch_prefill<T, 128, 1, false, MASKED, PAD>(p, stream);
@@ -406,6 +459,7 @@ static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, hipStr
 int prefill_rows64(const PrefillParams& p, bool causal, bool f16, void* ws, size_t ws_bytes, hipStream_t stream);
 bool prefill_rows64_fits(const PrefillParams& p);
 int prefill_rows64_spans(const PrefillParams& p, bool causal, bool f16, hipStream_t stream);
+bool prefill_rows64_streamk(const PrefillParams& p, bool causal, hipStream_t stream);
 size_t rows64_sk_workspace(const dtattn_prefill_args* a, int device);
 
 // Kernel head dim of a bf16/fp16 call: the smallest of 64, 128, 256, 512 holding both real head dims.
@@ -475,9 +529,39 @@ static size_t mask_rows_workspace(const dtattn_prefill_args* a, const dtattn_mas
     return (((size_t)*slabs * sizeof(int2) + 255) & ~(size_t)255) + (size_t)*slabs * *pitch * sizeof(float);
 }
 
+static int stream_device(hipStream_t stream, int* dev) {
+    return (stream == nullptr ? hipGetDevice(dev) : hipStreamGetDevice(stream, dev)) == hipSuccess ? DTATTN_OK
+                                                                                               : DTATTN_ERR_DEVICE;
+}
+
+// Key groups of prefill_fwd_kernel for a call without mask or padding, or 0: the grid is large enough for the kernels
+// with 64 rows per wave (head dim 128).  A workgroup ends no sooner than its own key tiles, and a 64-row wave takes
+// 1.35 us a tile against 0.95 us here, so up to two workgroups per CU 128-row blocks of one head end first (causal
+// 1x32/8x512 18.0 -> 13.8 us, 2x32/8x777 23.1 -> 20.4, 4x32/8x512 18.3 -> 15.8; 16x32/8x128 not causal 11.8 -> 9.5); a
+// non-causal grid of long rows is as good on the 64-row kernel already (1x32/8x1500 42.6 against 40.6).  Two key groups
+// halve the chain of tiles, for 128 KB of LDS at head dim 128 and a merge worth 1-2 us: from 8 tiles on, on grids of one
+// workgroup per CU (causal 1x32/8x1024 22.3 -> 20.9, 777 18.2 -> 16.7, 400 11.9 both; D = 64 1x12x1024 15.8 -> 13.4) and
+// on causal ones of two where the second round is the short blocks of many (1x32/8x1500 32.0 -> 28.8, D = 64 1x12x4096
+// 51.5 -> 39.7; of 7 blocks, 1x64/8x777, 20.1 -> 24.5).
+static int key_groups(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
+    int dev = 0;
+    dtattn_device_peaks pk;
+    if (stream_device(stream, &dev) != DTATTN_OK || dtattn_get_device_peaks(dev, &pk) != DTATTN_OK) return D == 128 ? 0 : 1;
+    const int64_t blocks = ((int64_t)p.Sq + 127) / 128, grid = blocks * p.B * p.Hq;
+    int64_t keys = p.Sk;  // of the longest workgroup
+    if (causal) keys = std::max<int64_t>(0, std::min<int64_t>(keys, (int64_t)p.Sq + p.delta));
+    const int64_t tiles = (keys + 63) / 64;
+    if (grid <= pk.cu_count) return tiles >= 8 ? 2 : 1;
+    if (grid <= 2 * pk.cu_count) {
+        if (causal) return tiles >= 8 && blocks >= 12 ? 2 : 1;
+        if (tiles <= 16) return 1;
+    }
+    return D == 128 ? 0 : 1;
+}
+
 // D is the kernel's head dim (64 or 128); pad: the real head dims are below it.  Head dim 128 without mask or
-// padding runs the 64-rows-per-wave kernel (prefill_rows64.hip), which returns the same bits as
-// prefill_fwd_kernel at 4-9% (non-causal) and 4-14% (causal) more throughput.
+// padding runs the 64-rows-per-wave kernel (prefill_rows64.hip) on grids that fill the chip, which returns the same
+// bits as prefill_fwd_kernel at 4-9% (non-causal) and 4-14% (causal) more throughput.
 template <typename T>
 static int dispatch_prefill(PrefillParams p, int D, bool causal, bool pad, void* ws, size_t ws_bytes, hipStream_t stream) {
     // Row masks with key spans: the batches that have one run as shorter calls without a mask, on the faster kernel
@@ -492,17 +576,22 @@ static int dispatch_prefill(PrefillParams p, int D, bool causal, bool pad, void*
             p.spans = nullptr;
         }
     }
-    if (D == 128 && !pad && p.mask == nullptr && prefill_rows64_fits(p))
-        return prefill_rows64(p, causal, __is_same(T, f16_t), ws, ws_bytes, stream);
+    int kg = 1;
+    if (!pad && p.mask == nullptr) {
+        const bool fits64 = D == 128 && prefill_rows64_fits(p);
+        kg = key_groups(p, D, causal, stream);
+        if (fits64 && (kg == 0 || prefill_rows64_streamk(p, causal, stream)))
+            return prefill_rows64(p, causal, __is_same(T, f16_t), ws, ws_bytes, stream);
+    }
     const MaskMode mode = mask_mode(p);
     auto run = [&](auto pad_c) {
         constexpr bool PAD = decltype(pad_c)::value;
         switch (mode) {
-            case kMaskF32: return dispatch_prefill_m<T, kMaskF32, PAD>(p, D, causal, stream);
-            case kMaskBool: return dispatch_prefill_m<T, kMaskBool, PAD>(p, D, causal, stream);
-            case kMaskBf16: return dispatch_prefill_m<T, kMaskBf16, PAD>(p, D, causal, stream);
-            case kMaskF16: return dispatch_prefill_m<T, kMaskF16, PAD>(p, D, causal, stream);
-            default: return dispatch_prefill_m<T, kMaskNone, PAD>(p, D, causal, stream);
+            case kMaskF32: return dispatch_prefill_m<T, kMaskF32, PAD>(p, D, causal, kg, stream);
+            case kMaskBool: return dispatch_prefill_m<T, kMaskBool, PAD>(p, D, causal, kg, stream);
+            case kMaskBf16: return dispatch_prefill_m<T, kMaskBf16, PAD>(p, D, causal, kg, stream);
+            case kMaskF16: return dispatch_prefill_m<T, kMaskF16, PAD>(p, D, causal, kg, stream);
+            default: return dispatch_prefill_m<T, kMaskNone, PAD>(p, D, causal, kg, stream);
         }
     };
     return pad ? run(std::true_type{}) : run(std::false_type{});
@@ -533,11 +622,6 @@ static int wide_plan(const dtattn_prefill_args* a, int device, size_t* bytes, si
     *lse_off = (o_bytes + 255) & ~(size_t)255;
     *bytes = *lse_off + (size_t)splits * a->B * a->Hq * a->Sq * sizeof(float);
     return splits;
-}
-
-static int stream_device(hipStream_t stream, int* dev) {
-    return (stream == nullptr ? hipGetDevice(dev) : hipStreamGetDevice(stream, dev)) == hipSuccess ? DTATTN_OK
-                                                                                               : DTATTN_ERR_DEVICE;
 }
 
 static int mask_element_size(int32_t dtype) {

@@ -918,23 +918,35 @@ static int launch_rows64_plain(const PrefillParams& p, bool gqa, hipStream_t str
     return launch_rows64<T, CAUSAL, CAUSAL ? 2 : 4, SPAN>(p, stream);
 }
 
-// ws / ws_bytes: the caller's workspace (may be NULL); non-causal row-layout calls whose grid would leave a
-// ragged last round take the stream-K form when it holds the records.
+// Whether the call has a stream-K form, its shares and the workspace its records need: non-causal calls whose grid
+// would leave a ragged last round.
+static bool sk_form(const PrefillParams& p, bool causal, hipStream_t stream, Rows64Sk* sk, size_t* need) {
+    const bool positive = p.q_and == 0xffffffffu && p.q_xor == 0u;
+    if (causal || !positive) return false;
+    int dev = 0;
+    dtattn_device_peaks pk;
+    return rows64_stream_device(stream, &dev) == DTATTN_OK && dtattn_get_device_peaks(dev, &pk) == DTATTN_OK &&
+           rows64_sk_plan(p.B, p.Hq, p.Sq, p.Sk, p.group >= 4 && p.group % 4 == 0, pk.cu_count, sk, need);
+}
+
+bool prefill_rows64_streamk(const PrefillParams& p, bool causal, hipStream_t stream) {
+    Rows64Sk sk;
+    size_t need = 0;
+    return sk_form(p, causal, stream, &sk, &need);
+}
+
+// ws / ws_bytes: the caller's workspace (may be NULL); calls with a stream-K form take it when this holds the records.
 int prefill_rows64(const PrefillParams& p, bool causal, bool f16, void* ws, size_t ws_bytes, hipStream_t stream) {
     const bool positive = p.q_and == 0xffffffffu && p.q_xor == 0u;
     const bool gqa_form = p.group >= 4 && p.group % 4 == 0;
-    if (!causal && positive && ws != nullptr && (reinterpret_cast<uintptr_t>(ws) & 255u) == 0) {
-        int dev = 0;
-        dtattn_device_peaks pk;
-        Rows64Sk sk;
-        size_t need = 0;
-        if (rows64_stream_device(stream, &dev) == DTATTN_OK && dtattn_get_device_peaks(dev, &pk) == DTATTN_OK &&
-            rows64_sk_plan(p.B, p.Hq, p.Sq, p.Sk, gqa_form, pk.cu_count, &sk, &need) && need <= ws_bytes) {
-            sk.ws = static_cast<char*>(ws);
-            if (gqa_form)
-                return f16 ? launch_rows64_sk<f16_t, true>(p, sk, stream) : launch_rows64_sk<bf16_t, true>(p, sk, stream);
-            return f16 ? launch_rows64_sk<f16_t, false>(p, sk, stream) : launch_rows64_sk<bf16_t, false>(p, sk, stream);
-        }
+    Rows64Sk sk;
+    size_t need = 0;
+    if (ws != nullptr && (reinterpret_cast<uintptr_t>(ws) & 255u) == 0 && sk_form(p, causal, stream, &sk, &need) &&
+        need <= ws_bytes) {
+        sk.ws = static_cast<char*>(ws);
+        if (gqa_form)
+            return f16 ? launch_rows64_sk<f16_t, true>(p, sk, stream) : launch_rows64_sk<bf16_t, true>(p, sk, stream);
+        return f16 ? launch_rows64_sk<f16_t, false>(p, sk, stream) : launch_rows64_sk<bf16_t, false>(p, sk, stream);
     }
     return f16 ? (causal ? launch_rows64_plain<f16_t, true, false>(p, gqa_form && positive, stream)
                          : launch_rows64_plain<f16_t, false, false>(p, gqa_form && positive, stream))
