@@ -17,39 +17,10 @@
 // writes back and invalidates the XCD's L2, which costs far more than the second launch.)
 #include <mutex>
 
+#include "decode_params.hpp"
 #include "dtattn_common.hpp"
 
 namespace dtattn {
-
-struct DecodeParams {
-    const void* q;
-    const void* k;
-    const void* v;
-    const int32_t* lengths;
-    void* o;
-    float* lse;
-    float* part_o;    // [B, Hq, nsplit, D]
-    float* part_lse;  // [B, Hq, nsplit]
-    int64_t qs_b, qs_h;
-    int64_t ks_b, ks_h, ks_s;
-    int64_t vs_b, vs_h, vs_s;
-    int64_t os_b, os_h;
-    int64_t lses_b;
-    int32_t B, Hq, Hkv, S_max, group;
-    int32_t chunk, nsplit;
-    float c;  // scale * log2(e)
-    // paged cache: token t of sequence b is row t & (2^page_shift - 1) of page
-    // block_table[b * bt_s + (t >> page_shift)]; ks_b / vs_b are then the page strides
-    const int32_t* block_table;
-    int64_t bt_s;
-    int32_t page_shift, num_pages;
-    // bytes from a kv head's base to the end of its last page row (K, V), when every page offset fits 32 bits
-    // (strides >= 0, span < 2^32): the paged loads then go through buffer resources; 0: 64-bit flat loads
-    uint32_t kspan, vspan;
-    // real head dim (<= the kernel's D; a multiple of 16 bytes of elements) and its 16-byte chunks
-    int32_t d_real, d_ch;
-    uint32_t q_and, q_xor;  // applied to q's words at load, as in ScalePlan
-};
 
 constexpr int kDecodeChunk = 128;  // smallest split; workspace queries with chunk 0 size for it
 
@@ -628,6 +599,8 @@ static int decode_splitkv_run(const dtattn_decode_args* a, void* ws, size_t ws_b
     p.page_shift = 0;
     p.num_pages = 0;
     p.kspan = p.vspan = 0;
+    p.d_real = (int32_t)a->D;
+    if (a->chunk <= 0 && decode_stream_fits(p, a->dtype, ws_bytes, stream)) return decode_stream(p, a->dtype, ws, stream);
     if (a->dtype == DTATTN_BF16) return dispatch_decode<bf16_t, 0>(p, (int)a->D, stream);
     if (a->dtype == DTATTN_FP32) return dispatch_decode<float, 0>(p, (int)a->D, stream);
     return dispatch_decode<f16_t, 0>(p, (int)a->D, stream);
@@ -729,6 +702,9 @@ extern "C" int dtattn_decode_paged(const dtattn_decode_paged_args* a, void* stre
     p.kspan = span(a->k_stride);
     p.vspan = span(a->v_stride);
     if (p.kspan == 0 || p.vspan == 0) p.kspan = p.vspan = 0;
+    p.d_real = (int32_t)a->D;
+    if (a->chunk <= 0 && decode_stream_fits(p, a->dtype, a->workspace_bytes, stream))
+        return decode_stream(p, a->dtype, a->workspace, stream);
     if (p.kspan != 0 && a->page_size == 16 && a->dtype != DTATTN_FP32) {
         if (a->dtype == DTATTN_BF16) return dispatch_decode<bf16_t, 3>(p, (int)a->D, stream);
         return dispatch_decode<f16_t, 3>(p, (int)a->D, stream);

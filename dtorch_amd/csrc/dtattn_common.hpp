@@ -194,6 +194,14 @@ __device__ __forceinline__ void buf_ld16_lds_async(__amdgpu_buffer_rsrc_t r, voi
                  : "s"(lds_addr), "v"(voffset), "s"(r)
                  : "m0");
 }
+// With the non-temporal hint, for data streamed exactly once.
+__device__ __forceinline__ void buf_ld16_lds_async_nt(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voffset) {
+    const uint32_t lds_addr = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                 :
+                 : "s"(lds_addr), "v"(voffset), "s"(r)
+                 : "m0");
+}
 #pragma clang diagnostic pop
 
 // ---- wave helpers -----------------------------------------------------------------------------

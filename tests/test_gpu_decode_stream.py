@@ -1,0 +1,77 @@
+"""The streaming decode (decode_stream.hip: larger bf16 / fp16 batches at head dim 128) against the split form and the
+oracle.
+
+An explicit chunk selects the split form, so both run on the same inputs.  Both keep scores, sums and partial outputs
+in fp32 and round P and O to the input type, over different splits: their O differ by those roundings (2^-9 of P and
+of |O| < 3 in bf16), the LSE by fp32 ones.  Lengths sit at the ends of a 32-token unit, of the 64 sequences a wave's
+prefix covers at once, and at zero; rows of the caches past a length hold NaN.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import sdpa as orc
+from tests.attn_cases import LSE_TOL, O_TOL_BF16, host, lse_rel, max_abs
+
+pytestmark = pytest.mark.gpu
+
+
+def _lengths(kind, B, cap, rng):
+    edge = [0, 1, 31, 32, 33, 63, 64, 65, cap - 1, cap]
+    if kind == "mixed":
+        n = np.concatenate([edge, rng.integers(0, cap + 1, B - len(edge))])
+        return rng.permutation(n)
+    if kind == "short":  # a share spans many sequences
+        return rng.integers(0, 40, B)
+    if kind == "one":  # every wave cuts the same sequence; the others are empty
+        return np.where(np.arange(B) == B - 1, cap, 0)
+    return np.ones(B, dtype=int)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,cap,page,kind,dtype,scale", [
+    (70, 8, 2, 1024, 0, "mixed", torch.bfloat16, None),
+    (70, 8, 2, 1024, 16, "mixed", torch.float16, None),
+    (70, 14, 2, 1024, 32, "mixed", torch.bfloat16, None),    # groups of 7
+    (130, 16, 2, 512, 64, "short", torch.bfloat16, -0.1),    # groups of 8, a negative scale
+    (33, 32, 32, 1024, 256, "mixed", torch.bfloat16, None),  # groups of 1
+    (70, 8, 2, 1024, 16, "one", torch.bfloat16, None),
+    (70, 8, 2, 1024, 0, "ones", torch.bfloat16, None),
+    (2, 10, 2, 16384, 0, "one", torch.float16, None),        # groups of 5; merged by four waves a head
+])
+def test_stream_against_split_and_oracle(B, Hq, Hkv, cap, page, kind, dtype, scale):
+    import dtorch_amd.nn.functional as F
+    D = 128
+    rng = np.random.default_rng(B + cap + page)
+    lens = _lengths(kind, B, cap, rng)
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q = torch.randn(B, Hkv, Hq // Hkv, D, device="cuda", generator=g).to(dtype).flatten(1, 2)[:, :, None]
+    # [B, S, H, D] storage: rows of a head are not contiguous
+    k, v = (torch.randn(B, cap, Hkv, D, device="cuda", generator=g).to(dtype).transpose(1, 2) for _ in range(2))
+    past = torch.arange(cap, device="cuda")[None, :] >= torch.tensor(lens, device="cuda")[:, None]
+    for t in (k, v):
+        t.masked_fill_(past[:, None, :, None], float("nan"))
+    tl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    if page:
+        per = cap // page
+        table = torch.randperm(B * per, device="cuda", generator=g).view(B, per)
+        pages = []
+        for t in (k, v):
+            pool = torch.empty(B * per, Hkv, page, D, dtype=dtype, device="cuda")
+            pool[table.flatten()] = t.unflatten(2, (per, page)).transpose(1, 2).flatten(0, 1)
+            pages.append(pool)
+        run = lambda chunk: F.decode_attention_paged(q, *pages, table.to(torch.int32), tl, scale=scale, chunk=chunk)
+    else:
+        run = lambda chunk: F.decode_attention(q, k, v, tl, scale=scale, chunk=chunk)
+    o, lse = run(0)
+    o2, lse2 = run(0)
+    os_, ls = run(384)
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    assert max_abs(host(o), host(os_)) <= O_TOL_BF16 and lse_rel(host(lse), host(ls)) <= 1e-5
+    for b in np.unique(np.concatenate([[0, B - 1], rng.integers(0, B, 6), np.flatnonzero(lens == lens.max())[:1]])):
+        n = int(lens[b])
+        if n == 0:
+            assert not o[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rl = orc.sdpa_fwd(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), scale=scale, enable_gqa=True)
+        assert max_abs(host(o[b:b + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[b:b + 1]), rl[:, :, 0]) <= LSE_TOL
