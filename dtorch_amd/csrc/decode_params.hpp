@@ -34,6 +34,8 @@ struct DecodeParams {
     uint32_t q_and, q_xor;  // applied to q's words at load, as in ScalePlan
 };
 
+// Whether a 16-bit call at head dim 128 is large enough for the streaming form.
+bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hipStream_t stream);
 // The streaming form (decode_stream.hip): whether a call on the current device takes it (its partials fit `ws_bytes`),
 // and its two launches.
 bool decode_stream_fits(const DecodeParams& p, int32_t dtype, size_t ws_bytes, hipStream_t stream);

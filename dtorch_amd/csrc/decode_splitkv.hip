@@ -30,8 +30,16 @@ constexpr int kDecodeChunk = 128;  // smallest split; workspace queries with chu
 // registers that 2 waves per SIMD leave free); 256 for fp32 rows.  Measured on one MI355X over batch
 // 1-128, contexts 2K-128K, 4 heads per workgroup: 384 was 1-8% faster than 256 at D = 64 and 128
 // everywhere except one 8K sequence (-1 to -2%); 256 had been best or within 2% of 128 and 512.
-static int32_t auto_chunk(int64_t Hq, int64_t Hkv, int64_t esz) {
-    if ((Hq / Hkv) % 8 == 0 && Hkv % 8 != 0) return 128;
+//
+// 16-bit calls at head dim 128 in groups of 3 to 8 heads that are too small for the streaming form take 128 as well: their
+// grids leave CUs idle, and a third of the bytes per workgroup ends sooner than the merge of three times the partials
+// costs (32 heads over 8, per call: 1x500 12.0 -> 8.2 us, 1x4000 12.4 -> 9.3, 4x1000 13.2 -> 8.9, 16x500 14.5 -> 11.9; 64
+// over 8: 1x4000 13.3 -> 12.5; 28 over 4: 1x1000 8.2 -> 6.9, 1x8000 15.4 -> 15.7, the one size it loses).  Where the
+// streaming form is out for another reason (a pool past 4 GB), 384 stays above that bound.
+static int32_t auto_chunk(int64_t B, int64_t Hq, int64_t Hkv, int64_t S_max, int64_t D, int64_t esz, hipStream_t stream) {
+    const int64_t group = Hq / Hkv;
+    if (group % 8 == 0 && Hkv % 8 != 0) return 128;
+    if (esz == 2 && D == 128 && group >= 3 && group <= 8 && !decode_stream_pays(B, Hkv, S_max, group, stream)) return 128;
     return esz == 2 ? 384 : 256;
 }
 
@@ -420,7 +428,7 @@ static int launch_decode(const DecodeParams& p, hipStream_t stream) {
     dim3 grid((unsigned)(p.Hkv * (p.group / G)), (unsigned)p.B, (unsigned)p.nsplit);
     hipLaunchKernelGGL((decode_kernel<T, D, G, TPW, PAGED>), grid, dim3(256), 0, stream, p);
     int st = check_launch("decode_kernel");
-    if (st != DTATTN_OK) return st;
+    if (st != DTATTN_OK || p.nsplit == 1) return st;  // one split: decode_kernel wrote the outputs
     const int64_t pairs = (int64_t)p.B * p.Hq;
     hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, stream, p);
     return check_launch("decode_merge_kernel");
@@ -536,7 +544,7 @@ static int decode_splitkv_run(const dtattn_decode_args* a, void* ws, size_t ws_b
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->Hq, a->Hkv, esz);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, a->S_max, a->D, esz, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode: chunk %d must be 128, 256, 384 or 512", chunk);
     // chunk rows are addressed with 32-bit byte offsets
@@ -641,7 +649,7 @@ extern "C" int dtattn_decode_paged(const dtattn_decode_paged_args* a, void* stre
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode_paged: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->Hq, a->Hkv, esz);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, S_max, a->D, esz, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode_paged: chunk %d must be 128, 256, 384 or 512", chunk);
     if (a->q == nullptr || a->k_pages == nullptr || a->v_pages == nullptr || a->block_table == nullptr ||

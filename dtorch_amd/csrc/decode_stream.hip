@@ -416,19 +416,24 @@ static int stream_shares(const DecodeParams& p, hipStream_t stream) {
     return (int)std::min<int64_t>(4 * (int64_t)stream_cus(stream), (int64_t)p.B * p.Hkv * ((p.S_max + 127) / 128) / 2);
 }
 
+// Units per CU from which it is faster, by the capacity (the host does not know the lengths).  Its fixed cost is about 2 us
+// above the split form's; that form reads a chunk twice for 8 heads and 7 times for 7, and keeps up longest where
+// every head reads its own cache (1: 16x1000 44.0 against 46.9 us, 16x2000 86.9 against 84.6; 4: 16x500 15.1 against
+// 16.4, 16x1000 21.7 against 17.9; 8: 4x1000 14.4 against 16.3, 16x500 19.7 against 16.5;
+// 7: 8x1000 13.4 against 15.9).
+bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hipStream_t stream) {
+    const int64_t per_cu = group >= 5 ? 6 : group >= 3 ? 15 : 124;
+    const int cus = stream_cus(stream);
+    return cus > 0 && B * Hkv * ((S_max + kUnit - 1) / kUnit) >= per_cu * cus;
+}
+
 bool decode_stream_fits(const DecodeParams& p, int32_t dtype, size_t ws_bytes, hipStream_t stream) {
     if ((dtype != DTATTN_BF16 && dtype != DTATTN_FP16) || p.d_real != kStreamD || p.group > kStreamHeads) return false;
     if (p.block_table != nullptr && (p.kspan == 0 || p.page_shift < 4)) return false;
     if ((reinterpret_cast<uintptr_t>(p.o) & 7u) != 0 || p.os_b % 4 != 0 || p.os_h % 4 != 0) return false;
     if (p.qs_h < 0 || p.qs_h * p.group >= (1 << 28) || p.ks_s < 0 || p.vs_s < 0) return false;
-    const int64_t units = (int64_t)p.B * p.Hkv * ((p.S_max + kUnit - 1) / kUnit);
-    if (units >= ((int64_t)1 << 31)) return false;
-    // Units per CU from which it is faster, by the capacity (the host does not know the lengths).  Its fixed cost is
-    // about 2 us above the split form's; that form reads a chunk twice for 8 heads and 7 times for 7, and keeps up
-    // longest where every head reads its own cache (1: 16x1000 44.0 against 46.9 us, 16x2000 86.9 against 84.6; 4:
-    // 16x500 15.1 against 16.4, 16x1000 21.7 against 17.9; 8: 4x1000 14.4 against 16.3, 16x500 19.7 against 16.5).
-    const int64_t per_cu = p.group >= 5 ? 6 : p.group >= 3 ? 15 : 124;
-    if (units < per_cu * stream_cus(stream)) return false;
+    if (!decode_stream_pays(p.B, p.Hkv, p.S_max, p.group, stream)) return false;
+    if ((int64_t)p.B * p.Hkv * ((p.S_max + kUnit - 1) / kUnit) >= ((int64_t)1 << 31)) return false;
     const int n = stream_shares(p, stream);
     return n > 0 && (size_t)(2 * n) * p.group * (kStreamD + 1) * sizeof(float) <= ws_bytes;
 }

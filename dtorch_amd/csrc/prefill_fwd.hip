@@ -508,18 +508,29 @@ __global__ void __launch_bounds__(256) mask_rows_kernel(const void* mask, int ki
     const int64_t off = (slab / heads) * ms_b + (slab % heads) * ms_h;
     float* row = rows + slab * pitch;
     int first = Sk, last = -1, count = 0, other = 0;
-    for (int j = threadIdx.x; j < Sk; j += 256) {
-        float m;
-        if (kind == DTATTN_BOOL) m = reinterpret_cast<const uint8_t*>(mask)[off + j] != 0 ? 0.f : kNegInf;
-        else if (kind == DTATTN_BF16) m = (float)reinterpret_cast<const bf16_t*>(mask)[off + j];
-        else if (kind == DTATTN_FP16) m = (float)reinterpret_cast<const f16_t*>(mask)[off + j];
-        else m = reinterpret_cast<const float*>(mask)[off + j];
-        row[j] = m;
-        if (m * inv_scale != kNegInf) {  // not hidden
-            first = min(first, j);
-            last = max(last, j);
-            ++count;
-            other |= m != 0.f;  // NaN too
+    constexpr int NB = 8;  // loads in flight: one memory latency per 2048 keys
+    for (int j0 = threadIdx.x; j0 < Sk; j0 += 256 * NB) {
+        float mv[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int64_t at = off + min(j0 + 256 * i, Sk - 1);
+            if (kind == DTATTN_BOOL) mv[i] = reinterpret_cast<const uint8_t*>(mask)[at] != 0 ? 0.f : kNegInf;
+            else if (kind == DTATTN_BF16) mv[i] = (float)reinterpret_cast<const bf16_t*>(mask)[at];
+            else if (kind == DTATTN_FP16) mv[i] = (float)reinterpret_cast<const f16_t*>(mask)[at];
+            else mv[i] = reinterpret_cast<const float*>(mask)[at];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int j = j0 + 256 * i;
+            if (j >= Sk) break;
+            const float m = mv[i];
+            row[j] = m;
+            if (m * inv_scale != kNegInf) {  // not hidden
+                first = min(first, j);
+                last = max(last, j);
+                ++count;
+                other |= m != 0.f;  // NaN too
+            }
         }
     }
 #pragma unroll

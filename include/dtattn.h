@@ -171,10 +171,11 @@ typedef struct {
     int32_t dtype;         /* BF16, FP16 or FP32 (FP32 from ABI version 5) */
     float scale;           /* NaN means 1/sqrt(D) (ABI version 8) */
     int32_t chunk;         /* tokens per split: 128, 256, 384 or 512; 0 picks 128 when Hq / Hkv is a
-                              multiple of 8 and Hkv is not, else 384 for bf16/fp16 and 256 for
-                              fp32, or, for larger bf16/fp16 batches at D = 128 and up to 8 heads
-                              per kv head, equal shares of all tokens instead of splits; workspace
-                              sizes for chunk 0 cover every choice */
+                              multiple of 8 and Hkv is not, and for small bf16/fp16 batches at
+                              D = 128 in groups of 3 to 8 heads, else 384 for bf16/fp16 and 256
+                              for fp32, or, for larger bf16/fp16 batches at D = 128 and up to 8
+                              heads per kv head, equal shares of all tokens instead of splits;
+                              workspace sizes for chunk 0 cover every choice */
     void* workspace;       /* >= dtattn_decode_workspace_size(...) bytes, 256-byte aligned */
     size_t workspace_bytes;
 } dtattn_decode_args;
