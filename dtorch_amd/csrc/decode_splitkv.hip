@@ -24,25 +24,6 @@ namespace dtattn {
 
 constexpr int kDecodeChunk = 128;  // smallest split; workspace queries with chunk 0 size for it
 
-// Split length picked for chunk = 0: 128 tokens for the 8-head workgroups (8 heads per workgroup
-// leave no registers for longer splits: 3.0 TB/s at 128 against 2.1-2.3 TB/s at 256); 384 for
-// 16-bit rows (each wave then keeps 1.5x the K/V bytes in flight of a 256-token split, using the
-// registers that 2 waves per SIMD leave free); 256 for fp32 rows.  Measured on one MI355X over batch
-// 1-128, contexts 2K-128K, 4 heads per workgroup: 384 was 1-8% faster than 256 at D = 64 and 128
-// everywhere except one 8K sequence (-1 to -2%); 256 had been best or within 2% of 128 and 512.
-//
-// 16-bit calls at head dim 128 in groups of 3 to 8 heads that are too small for the streaming form take 128 as well: their
-// grids leave CUs idle, and a third of the bytes per workgroup ends sooner than the merge of three times the partials
-// costs (32 heads over 8, per call: 1x500 12.0 -> 8.2 us, 1x4000 12.4 -> 9.3, 4x1000 13.2 -> 8.9, 16x500 14.5 -> 11.9; 64
-// over 8: 1x4000 13.3 -> 12.5; 28 over 4: 1x1000 8.2 -> 6.9, 1x8000 15.4 -> 15.7, the one size it loses).  Where the
-// streaming form is out for another reason (a pool past 4 GB), 384 stays above that bound.
-static int32_t auto_chunk(int64_t B, int64_t Hq, int64_t Hkv, int64_t S_max, int64_t D, int64_t esz, hipStream_t stream) {
-    const int64_t group = Hq / Hkv;
-    if (group % 8 == 0 && Hkv % 8 != 0) return 128;
-    if (esz == 2 && D == 128 && group >= 3 && group <= 8 && !decode_stream_pays(B, Hkv, S_max, group, stream)) return 128;
-    return esz == 2 ? 384 : 256;
-}
-
 // Kernel head dim for a real head dim: 64 or 128 (0: unsupported).  Smaller real dims run the
 // kernel of the next size, reading a valid chunk in place of each padded one with its query chunk
 // zeroed, so the padding adds nothing to the scores; the padded output columns are not stored.
@@ -55,6 +36,28 @@ size_t decode_ws_parts(int64_t B, int64_t Hq, int64_t S_max, int64_t D_real, int
     const size_t o_bytes = (size_t)B * Hq * nsplit * D * sizeof(float);
     const size_t lse_bytes = (size_t)B * Hq * nsplit * sizeof(float);
     return ((o_bytes + 255) & ~(size_t)255) + ((lse_bytes + 255) & ~(size_t)255);
+}
+
+// Split length picked for chunk = 0: 128 tokens for the 8-head workgroups (8 heads per workgroup
+// leave no registers for longer splits: 3.0 TB/s at 128 against 2.1-2.3 TB/s at 256); 384 for
+// 16-bit rows (each wave then keeps 1.5x the K/V bytes in flight of a 256-token split, using the
+// registers that 2 waves per SIMD leave free); 256 for fp32 rows.  Measured on one MI355X over batch
+// 1-128, contexts 2K-128K, 4 heads per workgroup: 384 was 1-8% faster than 256 at D = 64 and 128
+// everywhere except one 8K sequence (-1 to -2%); 256 had been best or within 2% of 128 and 512.
+//
+// 16-bit calls at head dim 128 in groups of 3 to 8 heads that are too small for the streaming form take 128 as well: their
+// grids leave CUs idle, and a third of the bytes per workgroup ends sooner than the merge of three times the partials
+// costs (32 heads over 8, per call: 1x500 12.0 -> 8.2 us, 1x4000 12.4 -> 9.3, 4x1000 13.2 -> 8.9, 16x500 14.5 -> 11.9; 64
+// over 8: 1x4000 13.3 -> 12.5; 28 over 4: 1x1000 8.2 -> 6.9, 1x8000 15.4 -> 15.7, the one size it loses).  Where the
+// streaming form is out for another reason (a pool past 4 GB), 384 stays above that bound.
+static int32_t auto_chunk(int64_t B, int64_t Hq, int64_t Hkv, int64_t S_max, int64_t D, int64_t esz, size_t ws_bytes,
+                          hipStream_t stream) {
+    const int64_t group = Hq / Hkv;
+    if (group % 8 == 0 && Hkv % 8 != 0) return 128;
+    if (esz == 2 && D == 128 && group >= 3 && group <= 8 && !decode_stream_pays(B, Hkv, S_max, group, stream) &&
+        decode_ws_parts(B, Hq, S_max, D, 128, nullptr) <= ws_bytes)  // a workspace sized for 384 keeps 384
+        return 128;
+    return esz == 2 ? 384 : 256;
 }
 
 // G heads per workgroup, D head dim, TPW tokens per wave (chunk = 4 * TPW, in sub-blocks per wave;
@@ -544,7 +547,7 @@ static int decode_splitkv_run(const dtattn_decode_args* a, void* ws, size_t ws_b
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, a->S_max, a->D, esz, stream);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, a->S_max, a->D, esz, noalloc ? kScratchBytes : ws_bytes, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode: chunk %d must be 128, 256, 384 or 512", chunk);
     // chunk rows are addressed with 32-bit byte offsets
@@ -649,7 +652,7 @@ extern "C" int dtattn_decode_paged(const dtattn_decode_paged_args* a, void* stre
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode_paged: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, S_max, a->D, esz, stream);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, S_max, a->D, esz, a->workspace_bytes, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode_paged: chunk %d must be 128, 256, 384 or 512", chunk);
     if (a->q == nullptr || a->k_pages == nullptr || a->v_pages == nullptr || a->block_table == nullptr ||

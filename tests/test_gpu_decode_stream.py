@@ -75,3 +75,24 @@ def test_stream_against_split_and_oracle(B, Hq, Hkv, cap, page, kind, dtype, sca
             continue
         ro, rl = orc.sdpa_fwd(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), scale=scale, enable_gqa=True)
         assert max_abs(host(o[b:b + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[b:b + 1]), rl[:, :, 0]) <= LSE_TOL
+
+
+@pytest.mark.parametrize("B,S", [(1, 4000), (70, 1024)])  # below and above the streaming form's line
+def test_smaller_workspace_is_still_accepted(B, S):
+    """chunk 0 with the workspace of 384-token splits, as 0 picked for these calls before it also picked 128."""
+    import ctypes
+    from tests.test_zz_no_alloc import BF16, _args, _case
+    from tests.test_zz_no_alloc import _lib as bound
+    lib = bound()
+    q, k, v, lengths = _case(B, 8, 2, S, 128, torch.bfloat16, B)
+    lengths.fill_(S - 3)
+    outs = []
+    for chunk in (0, 384):
+        o, lse = torch.empty_like(q), torch.empty(B, 8, device="cuda")
+        ws = torch.empty(lib.dtattn_decode_workspace_size(B, 8, S, 128, 384), dtype=torch.uint8, device="cuda")
+        a = _args(q, k, v, lengths, o, lse, BF16, chunk, ws)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert lib.dtattn_decode_splitkv(ctypes.byref(a), stream) == 0, lib.dtattn_last_error()
+        outs.append((host(o), host(lse)))
+    torch.cuda.synchronize()
+    assert max_abs(outs[0][0], outs[1][0]) <= O_TOL_BF16 and lse_rel(outs[0][1], outs[1][1]) <= 1e-5
