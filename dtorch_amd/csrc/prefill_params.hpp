@@ -103,10 +103,12 @@ struct MaskSlab {
     // s0..s3 += mask / scale
     __device__ __forceinline__ void add(Group g, float inv_scale, float& s0, float& s1, float& s2, float& s3) const {
         if constexpr (MODE == kMaskBool) {
-            // bit 0 of a byte, sign-extended and inverted, over -inf's bits: +0 or -inf
-            const int w = (int)bytes(g);
+            // Any non-zero byte keeps its key: bit 7 of `nz` says so for each byte (the sum cannot carry into the next
+            // one); sign-extended and inverted over -inf's bits it is +0 or -inf
+            const uint32_t w = bytes(g);
+            const int nz = (int)(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w);
             auto m = [](int keep) { return __builtin_bit_cast(float, (uint32_t)~keep & 0xff800000u); };
-            s0 += m(w << 31 >> 31), s1 += m(w << 23 >> 31), s2 += m(w << 15 >> 31), s3 += m(w << 7 >> 31);
+            s0 += m(nz << 24 >> 31), s1 += m(nz << 16 >> 31), s2 += m(nz << 8 >> 31), s3 += m(nz >> 31);
         } else if constexpr (MODE == kMaskF32) {
             const f32x4 m = __builtin_bit_cast(f32x4, g);
             s0 += m.x * inv_scale, s1 += m.y * inv_scale, s2 += m.z * inv_scale, s3 += m.w * inv_scale;

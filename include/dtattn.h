@@ -44,7 +44,7 @@ typedef enum {
     DTATTN_FP16 = 1,
     DTATTN_FP8_E4M3FN = 2, /* OCP e4m3fn, max 448, per-head descales */
     DTATTN_FP32 = 3,
-    DTATTN_BOOL = 4 /* attention masks only: one byte, 1 keeps a key, 0 hides it */
+    DTATTN_BOOL = 4 /* attention masks only: one byte, non-zero keeps a key, 0 hides it */
 } dtattn_dtype;
 
 /* Prefill / per-block attention: O = softmax(scale * Q K^T [causal]) V, plus the per-row LSE.
@@ -111,7 +111,7 @@ typedef struct {
 int dtattn_prefill_fwd(const dtattn_prefill_args* args, void* stream);
 
 /* dtattn_prefill_fwd with the attention mask as the caller holds it (ABI version 11; args->mask is NULL):
- * boolean (a byte of 1 keeps a key, 0 hides it), or added to the logits from bf16, fp16 or fp32.  Element
+ * boolean (a non-zero byte keeps a key, 0 hides it), or added to the logits from bf16, fp16 or fp32.  Element
  * (b, h, i, j) is data[b*stride[0] + h*stride[1] + i*stride[2] + j] (key stride 1, any strides >= 0, base aligned
  * to its elements).  Same results as the fp32 form of the same mask, without its conversion pass.  Head dims
  * up to 128 (D and Dv); BF16/FP16/FP32 inputs. */

@@ -67,3 +67,27 @@ def test_mask_dtypes(dtype, L, S, D, causal, start, pitch):
     o, lse = run(keep[:, :, :, :1].expand(B, 1, L, S).contiguous())
     got = run(keep[:, :, :, :1])
     assert torch.equal(got[0], o) and torch.equal(got[1], lse)
+
+
+@pytest.mark.parametrize("dtype,B,Hq,L,S,D,causal", [
+    (torch.bfloat16, 2, 4, 130, 97, 64, True),
+    (torch.float16, 2, 4, 77, 200, 128, False),
+    (torch.bfloat16, 8, 8, 1024, 1501, 128, True),   # one row for all queries: read once into fp32 rows
+    (torch.bfloat16, 1, 2, 33, 70, 256, False),      # wide heads: converted first
+    (torch.float32, 1, 2, 90, 100, 64, False),       # key-split fp32 form
+    (torch.float32, 4, 192, 200, 300, 64, True),     # 128-row fp32 form
+])
+def test_bool_bytes(dtype, B, Hq, L, S, D, causal):
+    """Bytes of a bool mask other than 0 and 1 (a uint8 tensor viewed as bool): any non-zero byte keeps its key."""
+    import dtorch_amd.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(L + S)
+    q, k, v = (torch.randn(B, h, n, D, device="cuda", generator=g).to(dtype) for h, n in ((Hq, L), (Hq // 2, S), (Hq // 2, S)))
+    rows = 1 if L == 1024 else L
+    at = torch.randint(0, 7, (B, 1, rows, S), device="cuda", generator=g)
+    raw = torch.tensor([0, 1, 2, 4, 128, 254, 255], dtype=torch.uint8, device="cuda")[at]
+    raw[0, :, 0, :64] = 255   # a tile that every byte keeps
+    kw = dict(is_causal=causal, enable_gqa=True)
+    o, lse = F.scaled_dot_product_attention_with_lse(q, k, v, attn_mask=raw.view(torch.bool), **kw)
+    ro, rl = F.scaled_dot_product_attention_with_lse(q, k, v, attn_mask=raw != 0, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(o, ro) and torch.equal(lse, rl)
