@@ -202,6 +202,27 @@ at::Tensor MaskView(const at::Tensor& m_, const at::Tensor& q, const at::Tensor&
     return e;
 }
 
+// Whether a mask is read as it is stored or converted to fp32 first.  us, as stored / converted, 32 query heads:
+//   a row of keys, fp16 and bf16, not causal: D = 128 2x1000 45 / 40, 4x2000 298 / 272; D = 64 2x1000 24.4 / 25.4, 4x1000
+//     48 / 51, 4x2000 178 / 160; causal: D = 128 4x1000 68 / 72, 4x2000 219 / 222; D = 64 2x1000 22.6 / 26.7, 4x1000 34 / 32,
+//     4x2000 108 / 95
+//   a row of keys, boolean, not causal: D = 128 4x1000 77 / 77, 4x2000 281 / 274; D = 64 4x1000 53 / 54, 2x2000 99 / 96,
+//     2x4000 331 / 304; causal: D = 128 4x2000 209 / 226, D = 64 4x2000 96 / 96
+//   a row per query, fp16 and bf16, D = 128, not causal: 1x1800 (2^26.6 pairs) 80 / 80, 1x2200 (2^27.2) 160 / 155, 2x2000
+//     184 / 170, 4x2000 365 / 344; causal: 1x1800 86 / 94, 4x2000 278 / 320
+bool StoredMaskPays(const at::Tensor& m, c10::ScalarType st, const View4& q, int64_t Sk, int64_t Dv, bool causal) {
+    const bool boolean = m.scalar_type() == at::kBool;
+    if (st == at::kFloat || (!boolean && m.scalar_type() != at::kBFloat16 && m.scalar_type() != at::kHalf)) return true;
+    const bool wide = std::max(q.D, Dv) > 64;
+    const double pairs = (double)q.B * (double)q.H * (double)q.S * (double)Sk;
+    const double ops = (wide ? 512.0 : 256.0) * pairs * (causal ? 0.5 : 1.0);
+    if (m.dim() < 2 || m.size(-2) == 1) {
+        if (boolean) return causal || ops < 4.5e10;
+        return causal ? wide || ops < 1.2e10 : ops < 2.4e10;
+    }
+    return boolean || causal || !wide || pairs < (double)((int64_t)1 << 27);
+}
+
 PrefillResult RunPrefill(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const SdpaParam& prm,
                          int64_t qOffset, int64_t kOffset, bool wantLse, const at::Tensor* mask = nullptr) {
     CheckDevice({&q_, &k_, &v_});
@@ -279,28 +300,7 @@ PrefillResult RunPrefill(const at::Tensor& q_, const at::Tensor& k_, const at::T
     a.scale = prm.scale.has_value() ? (float)prm.scale.value() : std::nanf("");  // NaN: 1/sqrt(D)
     a.causal = prm.isCausal ? 1 : 0;
     a.q_offset = qOffset, a.k_offset = kOffset;
-    at::Tensor maskt;
-    dtattn_mask mk;
-    // Masks go to the kernels as stored, but for wide heads (fp32 masks only) and large non-causal head-dim-128
-    // calls with a 16-bit mask of a row per query, where decoding it in the kernel costs more than converting it
-    // once (4x32x2000x2000: 373 against 339 us with the conversion).
-    bool maskAsStored = mask != nullptr && std::max(q.D, v.D) <= 128 && k.S > 0;
-    if (maskAsStored && !prm.isCausal && std::max(q.D, v.D) > 64 && st != at::kFloat &&
-        (mask->scalar_type() == at::kBFloat16 || mask->scalar_type() == at::kHalf) && mask->dim() >= 2 &&
-        mask->size(-2) > 1 && q.B * q.H * q.S * k.S >= ((int64_t)1 << 27))
-        maskAsStored = false;
-    if (mask != nullptr) {
-        if (fp8) Throw("attn_mask is not supported with sage_attn_type 'native_fp8'");
-        maskt = maskAsStored ? MaskView(*mask, q_, k_, q.B, q.H, q.S, k.S) : PrepareMask(*mask, q_, k_, q.B, q.H, q.S, k.S);
-        int64_t* ms = maskAsStored ? mk.stride : a.mask_stride;
-        for (int i = 0; i < 3; ++i) ms[i] = maskt.size(i) > 1 ? maskt.stride(i) : 0;
-        if (maskAsStored) {
-            mk.data = maskt.data_ptr();
-            mk.dtype = maskt.scalar_type() == at::kBool ? DTATTN_BOOL : DtypeCode(maskt.scalar_type());
-        } else {
-            a.mask = maskt.data_ptr<float>();
-        }
-    }
+    if (mask != nullptr && fp8) Throw("attn_mask is not supported with sage_attn_type 'native_fp8'");
 
     a.q = q.t.data_ptr(), a.k = k.t.data_ptr(), a.v = v.t.data_ptr();
     a.q_stride[0] = q.sb, a.q_stride[1] = q.sh, a.q_stride[2] = q.ss;
@@ -344,10 +344,37 @@ PrefillResult RunPrefill(const at::Tensor& q_, const at::Tensor& k_, const at::T
         if (!ov.t.is_same(o)) o.copy_(ov.t);
         return {o, lse};
     }
-    // Workspace for the key blocks of small wide-head grids, stream-K records or a padding mask's rows (zero bytes
-    // for every other call).
-    at::Tensor wst;
-    const size_t ws = maskAsStored ? dtattn_prefill_masked_workspace_size(&a, &mk) : dtattn_prefill_workspace_size(&a);
+    // Masks go to the kernels as stored, but for wide heads (fp32 masks only) and larger calls whose mask is small beside
+    // the scores, where decoding it for every query costs more than converting it once: 16-bit and boolean rows of keys
+    // (unless the call finds their spans, and converts them itself), and not causal 16-bit masks that the heads share.
+    // The workspace holds the key blocks of small wide-head grids, stream-K records or a padding mask's spans (zero bytes for
+    // every other call).
+    at::Tensor maskt, wst;
+    dtattn_mask mk;
+    bool maskAsStored = mask != nullptr && std::max(q.D, v.D) <= 128 && k.S > 0;
+    size_t ws = 0;
+    if (maskAsStored) {
+        auto view = [&](const at::Tensor& m) {
+            maskt = MaskView(m, q_, k_, q.B, q.H, q.S, k.S);
+            for (int i = 0; i < 3; ++i) mk.stride[i] = maskt.size(i) > 1 ? maskt.stride(i) : 0;
+            mk.data = maskt.data_ptr();
+            mk.dtype = maskt.scalar_type() == at::kBool ? DTATTN_BOOL : DtypeCode(maskt.scalar_type());
+            ws = dtattn_prefill_masked_workspace_size(&a, &mk);
+        };
+        view(*mask);
+        if (ws == 0 && !StoredMaskPays(*mask, st, q, k.S, v.D, prm.isCausal)) {
+            if (mask->dim() >= 2 && mask->size(-2) > 1)
+                maskAsStored = false;
+            else
+                view(mask->scalar_type() == at::kBool ? mask->to(at::kFloat).log_() : mask->to(at::kFloat));  // bool: 0, -inf
+        }
+    }
+    if (mask != nullptr && !maskAsStored) {
+        maskt = PrepareMask(*mask, q_, k_, q.B, q.H, q.S, k.S);
+        a.mask = maskt.data_ptr<float>();
+        for (int i = 0; i < 3; ++i) a.mask_stride[i] = maskt.size(i) > 1 ? maskt.stride(i) : 0;
+    }
+    if (!maskAsStored) ws = dtattn_prefill_workspace_size(&a);
     if (ws > 0) {
         wst = at::empty({(int64_t)ws}, q_.options().dtype(at::kByte));
         a.workspace = wst.data_ptr();

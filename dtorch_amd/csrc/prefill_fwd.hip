@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel
 
     const BlockCoord bc = block_coord<CAUSAL>(p);
     const int qb = bc.qb, b = bc.b, hq = bc.hq, hk = bc.hk;
-    if constexpr (MASKED == kMaskF32)
+    if constexpr (MASKED != kMaskNone)
         if (p.spans != nullptr && p.spans[b].y >= 0) return;  // run as a key span (prefill_rows64.hip)
 
     const T* qp = reinterpret_cast<const T*>(p.q) + b * p.qs_b + hq * p.qs_h;
@@ -497,16 +497,13 @@ static int kernel_head_dim(int64_t D, int64_t Dv) {
     return dmax <= 64 ? 64 : dmax <= 128 ? 128 : dmax <= 256 ? 256 : dmax <= 512 ? 512 : 0;
 }
 
-// A mask that is one row of keys per (batch, or batch and head), read once: the row in fp32 at rows + slab * pitch
-// (0 and -inf for a bool mask), which the attention kernels then read for every query without decoding it
-// again, and its key span (PrefillParams::spans).  One workgroup per slab; the row is a few KB, so this is one
-// short launch (about 3 us) ahead of a call of 40 us or more.
-__global__ void __launch_bounds__(256) mask_rows_kernel(const void* mask, int kind, int64_t ms_b, int64_t ms_h, int heads,
-                                                        int Sk, float inv_scale, float* rows, int64_t pitch, int2* spans) {
+// The key span of each batch (PrefillParams::spans) of a mask that is one row of keys for all queries and heads, and,
+// unless `rows` is NULL, that row in fp32 (0 and -inf for a bool mask) at rows + batch * pitch.  One workgroup per batch;
+// the row is a few KB, so this is one short launch ahead of a call of 40 us or more.
+__global__ void __launch_bounds__(256) mask_spans_kernel(const void* mask, int kind, int64_t ms_b, int Sk, float inv_scale,
+                                                         int2* spans, float* rows, int64_t pitch) {
     __shared__ int red[4][4];
-    const int slab = blockIdx.x;
-    const int64_t off = (slab / heads) * ms_b + (slab % heads) * ms_h;
-    float* row = rows + slab * pitch;
+    const int64_t off = (int64_t)blockIdx.x * ms_b;
     int first = Sk, last = -1, count = 0, other = 0;
     constexpr int NB = 8;  // loads in flight: one memory latency per 2048 keys
     for (int j0 = threadIdx.x; j0 < Sk; j0 += 256 * NB) {
@@ -524,7 +521,7 @@ __global__ void __launch_bounds__(256) mask_rows_kernel(const void* mask, int ki
             const int j = j0 + 256 * i;
             if (j >= Sk) break;
             const float m = mv[i];
-            row[j] = m;
+            if (rows != nullptr) rows[blockIdx.x * pitch + j] = m;
             if (m * inv_scale != kNegInf) {  // not hidden
                 first = min(first, j);
                 last = max(last, j);
@@ -550,23 +547,37 @@ __global__ void __launch_bounds__(256) mask_rows_kernel(const void* mask, int ki
         count += red[2][i];
         other |= red[3][i];
     }
-    spans[slab] = count == 0 ? make_int2(0, 0) : other == 0 && count == last + 1 - first ? make_int2(first, last + 1) : make_int2(0, -1);
+    spans[blockIdx.x] = count == 0 ? make_int2(0, 0)
+                        : other == 0 && count == last + 1 - first ? make_int2(first, last + 1) : make_int2(0, -1);
 }
 
-// Whether mask_rows_kernel runs ahead of a masked call, and the workspace it needs: bf16 / fp16 calls at kernel head
-// dims 64 and 128 whose mask is the same for every query, once they hold 2.4e10 operations (40 us and up at the
-// masked kernels' rate).  Below that its launch costs more than decoding the mask in the attention kernel.
-static size_t mask_rows_workspace(const dtattn_prefill_args* a, const dtattn_mask* mk, int64_t* pitch, int64_t* slabs) {
-    if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16) return 0;
-    if (a->B <= 0 || a->Hq <= 0 || a->Sq <= 1 || a->Sk <= 0 || mk->stride[2] != 0) return 0;
-    const int Dk = kernel_head_dim(a->D, a->Dv);
-    if (Dk != 64 && Dk != 128) return 0;
-    const double pairs = (double)a->B * (double)a->Hq * (double)a->Sq * (double)a->Sk * (a->causal != 0 ? 0.5 : 1.0);
-    if (4.0 * Dk * pairs < 2.4e10) return 0;
-    *slabs = a->B * (mk->stride[1] == 0 ? 1 : a->Hq);
-    *pitch = (a->Sk + 3) / 4 * 4;
-    if (*slabs > 0x7fffffff) return 0;
-    return (((size_t)*slabs * sizeof(int2) + 255) & ~(size_t)255) + (size_t)*slabs * *pitch * sizeof(float);
+// Whether mask_spans_kernel runs ahead of a masked call, and the workspace it needs: bf16 / fp16 calls at D = Dv = 128
+// (the span kernel's) whose mask is the same for every query and head, from 2.4e10 operations on, not causal from 3e10.
+// A call none of whose batches has a span pays 5-7 us for the two launches that find that out.  us without spans, with
+// them for left padding up to half, with them for a mask with a hole: causal 4x32/8x850 (2.4e10) 53, 35, 62, not causal
+// 8x32/8x400 (2.1e10) 40, 36, 43, 4x32/8x600 (2.4e10) 40, 41, 45, 4x32/8x700 (3.2e10) 49, 45, 50, 4x32/8x850 (4.7e10)
+// 64, 51, 67; causal 4x32/8x1000 65, 40, 72 (bool) and 67, 40, 72 (fp32).
+//
+// Not causal, batches without a span read a 16-bit or bool mask from fp32 rows (4x32/8x2000 bool 280 -> 270 us, bf16
+// 298 -> 270); causal they read it as stored (bool 226 -> 209, bf16 225 -> 219), and fp32 masks always (2x32/8x1000 42 -> 36).
+struct MaskSpans {
+    size_t bytes = 0, rows = 0;  // of the workspace; where the rows start, or 0
+    int64_t pitch = 0;           // of the rows, in elements
+};
+static MaskSpans mask_spans_plan(const dtattn_prefill_args* a, const dtattn_mask* mk) {
+    MaskSpans m;
+    if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16) return m;
+    if (a->B <= 0 || a->B > 0x7fffffff || a->Hq <= 0 || a->Sq <= 1 || a->Sk <= 0 || a->D != 128 || a->Dv != 128) return m;
+    if (mk->stride[1] != 0 || mk->stride[2] != 0) return m;
+    const double ops = 512.0 * (double)a->B * (double)a->Hq * (double)a->Sq * (double)a->Sk * (a->causal != 0 ? 0.5 : 1.0);
+    if (ops < (a->causal != 0 ? 2.4e10 : 3e10)) return m;
+    m.bytes = (size_t)a->B * sizeof(int2);
+    if (a->causal == 0 && mk->dtype != DTATTN_FP32) {
+        m.rows = (m.bytes + 255) & ~(size_t)255;
+        m.pitch = (a->Sk + 3) / 4 * 4;
+        m.bytes = m.rows + (size_t)a->B * m.pitch * sizeof(float);
+    }
+    return m;
 }
 
 static int stream_device(hipStream_t stream, int* dev) {
@@ -604,17 +615,12 @@ static int key_groups(const PrefillParams& p, int D, bool causal, hipStream_t st
 // bits as prefill_fwd_kernel at 4-9% (non-causal) and 4-14% (causal) more throughput.
 template <typename T>
 static int dispatch_prefill(PrefillParams p, int D, bool causal, bool pad, void* ws, size_t ws_bytes, hipStream_t stream) {
-    // Row masks with key spans: the batches that have one run as shorter calls without a mask, on the faster kernel
-    // and without the hidden tiles; prefill_fwd_kernel then runs the others and leaves at once for these (about 4 us
-    // of a call).  4x32/8x2000, left padding up to half: causal 219 -> 103 us, not causal 264 -> 186 us; a mask with
-    // holes 219 -> 222 us.
+    // Row masks with key spans (head dim 128): the batches that have one run as shorter calls without a mask, on the
+    // faster kernel and without the hidden tiles; prefill_fwd_kernel then runs the others and leaves at once for these
+    // (about 4 us of a call).  4x32/8x2000, left padding up to half: causal 219 -> 103 us, not causal 264 -> 186 us.
     if (p.spans != nullptr) {
-        if (D == 128 && !pad && p.ms_h == 0 && prefill_rows64_fits(p)) {
-            const int st = prefill_rows64_spans(p, causal, __is_same(T, f16_t), stream);
-            if (st != DTATTN_OK) return st;
-        } else {
-            p.spans = nullptr;
-        }
+        const int st = prefill_rows64_spans(p, causal, __is_same(T, f16_t), stream);
+        if (st != DTATTN_OK) return st;
     }
     int kg = 1;
     if (!pad && p.mask == nullptr) {
@@ -813,20 +819,20 @@ static int prefill_entry(const dtattn_prefill_args* a, const dtattn_mask* mk, vo
     p.q_xor = sp.q_xor;
     const bool causal = a->causal != 0;
     if (mk != nullptr && a->workspace != nullptr && (reinterpret_cast<uintptr_t>(a->workspace) & 255u) == 0) {
-        int64_t pitch = 0, slabs = 0;
-        const size_t need = mask_rows_workspace(a, mk, &pitch, &slabs);
-        if (need > 0 && need <= a->workspace_bytes) {
-            const int heads = (int)(slabs / a->B);
+        const MaskSpans m = mask_spans_plan(a, mk);
+        if (m.bytes > 0 && m.bytes <= a->workspace_bytes && prefill_rows64_fits(p)) {
             int2* spans = reinterpret_cast<int2*>(a->workspace);
-            float* rows = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + (((size_t)slabs * sizeof(int2) + 255) & ~(size_t)255));
-            hipLaunchKernelGGL(mask_rows_kernel, dim3((unsigned)slabs), dim3(256), 0, stream, mk->data, mk->dtype, mk->stride[0],
-                               mk->stride[1], heads, p.Sk, p.inv_scale, rows, pitch, spans);
-            const int st = check_launch("mask_rows_kernel");
+            float* rows = m.rows > 0 ? reinterpret_cast<float*>(static_cast<char*>(a->workspace) + m.rows) : nullptr;
+            hipLaunchKernelGGL(mask_spans_kernel, dim3((unsigned)a->B), dim3(256), 0, stream, mk->data, mk->dtype,
+                               mk->stride[0], p.Sk, p.inv_scale, spans, rows, m.pitch);
+            const int st = check_launch("mask_spans_kernel");
             if (st != DTATTN_OK) return st;
-            p.mask = rows;
-            p.mask_kind = DTATTN_FP32;
-            p.ms_b = heads * pitch, p.ms_h = heads > 1 ? pitch : 0, p.ms_l = 0;
             p.spans = spans;
+            if (rows != nullptr) {
+                p.mask = rows;
+                p.mask_kind = DTATTN_FP32;
+                p.ms_b = m.pitch;
+            }
         }
     }
     if (a->dtype == DTATTN_FP32) {
@@ -898,9 +904,7 @@ extern "C" int dtattn_prefill_masked(const dtattn_prefill_args* a, const dtattn_
 }
 
 extern "C" size_t dtattn_prefill_masked_workspace_size(const dtattn_prefill_args* a, const dtattn_mask* mask) {
-    if (a == nullptr || mask == nullptr) return 0;
-    int64_t pitch = 0, slabs = 0;
-    return mask_rows_workspace(a, mask, &pitch, &slabs);
+    return a == nullptr || mask == nullptr ? 0 : mask_spans_plan(a, mask).bytes;
 }
 
 extern "C" size_t dtattn_prefill_workspace_size(const dtattn_prefill_args* a) {

@@ -30,7 +30,7 @@ struct PrefillParams {
     const void* mask;
     int64_t ms_b, ms_h, ms_l;
     int32_t mask_kind;
-    // Key spans of a mask that is one row for all queries and heads (mask_rows_kernel), or NULL: entry b is the
+    // Key spans of a mask that is one row for all queries and heads (mask_spans_kernel), or NULL: entry b is the
     // [first, last + 1) visible keys of batch b when the mask hides every key outside and adds nothing inside,
     // else (0, -1).  The head-dim-128 kernels run the first kind as shorter calls, prefill_fwd_kernel the rest.
     const int2* spans;

@@ -122,10 +122,9 @@ typedef struct {
 } dtattn_mask;
 
 int dtattn_prefill_masked(const dtattn_prefill_args* args, const dtattn_mask* mask, void* stream);
-/* Workspace bytes (optional, 256-byte aligned) dtattn_prefill_masked can use: a large call whose mask is the same for
- * every query (a padding mask) first reads the mask once into fp32 rows and finds each batch's span of visible
- * keys.  Where the mask hides every key outside one span and adds nothing inside it, the keys outside are not read
- * at all. */
+/* Workspace bytes (optional, 256-byte aligned) dtattn_prefill_masked can use: a large BF16/FP16 call at D = Dv = 128
+ * whose mask is the same for every query and head (a padding mask) first finds each batch's span of visible keys.  Where
+ * the mask hides every key outside one span and adds nothing inside it, the keys outside are not read at all. */
 size_t dtattn_prefill_masked_workspace_size(const dtattn_prefill_args* args, const dtattn_mask* mask);
 /* Workspace bytes dtattn_prefill_fwd can use for `args` on the current device (0 when it would not
  * split the keys); 256-byte aligned pointers expected. */
