@@ -208,8 +208,9 @@ at::Tensor MaskView(const at::Tensor& m_, const at::Tensor& q, const at::Tensor&
 //     4x2000 108 / 95
 //   a row of keys, boolean, not causal: D = 128 4x1000 77 / 77, 4x2000 281 / 274; D = 64 4x1000 53 / 54, 2x2000 99 / 96,
 //     2x4000 331 / 304; causal: D = 128 4x2000 209 / 226, D = 64 4x2000 96 / 96
-//   a row per query, fp16 and bf16, D = 128, not causal: 1x1800 (2^26.6 pairs) 80 / 80, 1x2200 (2^27.2) 160 / 155, 2x2000
-//     184 / 170, 4x2000 365 / 344; causal: 1x1800 86 / 94, 4x2000 278 / 320
+//   a row per query, fp16 and bf16, D = 128, not causal, one for all heads: 1x1800 (2^26.6 pairs) 80 / 80, 1x2200 (2^27.2)
+//     160 / 155, 2x2000 184 / 170, 4x2000 365 / 344; one per head: 1x1800 94 / 257, 4x2000 534 / 1141; causal, one for
+//     all heads: 1x1800 86 / 94, 4x2000 278 / 320
 bool StoredMaskPays(const at::Tensor& m, c10::ScalarType st, const View4& q, int64_t Sk, int64_t Dv, bool causal) {
     const bool boolean = m.scalar_type() == at::kBool;
     if (st == at::kFloat || (!boolean && m.scalar_type() != at::kBFloat16 && m.scalar_type() != at::kHalf)) return true;
@@ -220,7 +221,7 @@ bool StoredMaskPays(const at::Tensor& m, c10::ScalarType st, const View4& q, int
         if (boolean) return causal || ops < 4.5e10;
         return causal ? wide || ops < 1.2e10 : ops < 2.4e10;
     }
-    return boolean || causal || !wide || pairs < (double)((int64_t)1 << 27);
+    return boolean || causal || !wide || (m.dim() >= 3 && m.size(-3) > 1) || pairs < (double)((int64_t)1 << 27);
 }
 
 PrefillResult RunPrefill(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const SdpaParam& prm,

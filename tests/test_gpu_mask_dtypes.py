@@ -91,3 +91,19 @@ def test_bool_bytes(dtype, B, Hq, L, S, D, causal):
     ro, rl = F.scaled_dot_product_attention_with_lse(q, k, v, attn_mask=raw != 0, **kw)
     torch.cuda.synchronize()
     assert torch.equal(o, ro) and torch.equal(lse, rl)
+
+
+@pytest.mark.parametrize("heads", [1, 16])
+def test_large_mask_of_a_row_per_query(heads):
+    """Not causal at D = 128 from 2^27 pairs on: a mask that the heads share is converted first, one per head is not."""
+    import dtorch_amd.nn.functional as F
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    H, S = 16, 2900
+    assert H * S * S >= 2 ** 27
+    q, k, v = (torch.randn(1, h, S, 128, device="cuda", generator=g).to(torch.bfloat16) for h in (H, 4, 4))
+    m = torch.randn(1, heads, S, S, device="cuda", generator=g).to(torch.bfloat16)
+    m.masked_fill_(torch.rand(m.shape, device="cuda", generator=g) < 0.2, float("-inf"))
+    o, lse = F.scaled_dot_product_attention_with_lse(q, k, v, attn_mask=m, enable_gqa=True)
+    ro, rl = F.scaled_dot_product_attention_with_lse(q, k, v, attn_mask=m.float(), enable_gqa=True)
+    torch.cuda.synchronize()
+    assert torch.equal(o, ro) and torch.equal(lse, rl)
