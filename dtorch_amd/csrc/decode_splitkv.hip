@@ -365,7 +365,8 @@ __global__ void __launch_bounds__(256) decode_kernel(const DecodeParams p) {
             if (d < p.d_real) obase[hq * p.os_h + d] = Elem<T>::from_f32(val / Lsum);
             if (p.lse != nullptr && d == 0) p.lse[b * p.lses_b + hq] = (M + __log2f(Lsum)) * kLn2;
         } else {
-            p.part_o[(((int64_t)b * p.Hq + hq) * p.nsplit + split) * D + d] = val / Lsum;
+            // every score -inf: O = 0, not 0 / 0, at the LSE of -inf that drops it in the merge
+            p.part_o[(((int64_t)b * p.Hq + hq) * p.nsplit + split) * D + d] = Lsum == 0.f ? 0.f : val / Lsum;
             if (d == 0) p.part_lse[((int64_t)b * p.Hq + hq) * p.nsplit + split] = (M + __log2f(Lsum)) * kLn2;
         }
     }

@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(64, 1) decode_stream_kernel(const DecodeParams
         const bool ends = left <= kUnit;  // the sequence's last unit
         if (ends || s + 1 == n) {
             const float lt = sum_across_groups<16>(l);
-            const float inv = 1.f / (lt * fast_exp2(M - m));
+            float inv = 1.f / (lt * fast_exp2(M - m));
             if (col < G) {
                 const int hq = cur.hk * G + col;
                 const float lse = __builtin_fmaf(M, kLn2, __log2f(lt) * kLn2);
@@ -318,6 +318,7 @@ __global__ void __launch_bounds__(64, 1) decode_stream_kernel(const DecodeParams
                     if (p.lse != nullptr && g4 == 0) p.lse[cur.b * p.lses_b + hq] = lse;
                 } else {
                     const int64_t rec = (int64_t)(2 * r + (cut_first ? 0 : 1)) * G + col;
+                    if (lt == 0.f) inv = 0.f;  // every score is -inf: O = 0, not 0 / 0, at the LSE of -inf that drops it
 #pragma unroll
                     for (int dt = 0; dt < 8; ++dt)
                         *reinterpret_cast<f32x4*>(p.part_o + rec * D + 16 * dt + 4 * g4) = acc[dt] * inv;

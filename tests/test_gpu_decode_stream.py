@@ -96,3 +96,31 @@ def test_smaller_workspace_is_still_accepted(B, S):
         outs.append((host(o), host(lse)))
     torch.cuda.synchronize()
     assert max_abs(outs[0][0], outs[1][0]) <= O_TOL_BF16 and lse_rel(outs[0][1], outs[1][1]) <= 1e-5
+
+
+@pytest.mark.parametrize("chunk", [0, 128, 384])  # streaming form, then splits
+@pytest.mark.parametrize("page", [0, 16])
+def test_parts_whose_scores_are_all_minus_infinity(page, chunk):
+    """Keys of -inf in a coordinate where every query is positive have a score of -inf, hence no weight, also where a
+    whole share or split holds nothing else; a part without weight adds nothing to the merge."""
+    import dtorch_amd.nn.functional as F
+    B, Hq, Hkv, cap, D, dtype = 70, 8, 2, 1024, 128, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(page + chunk)
+    q = torch.randn(B, Hq, 1, D, device="cuda", generator=g).to(dtype)
+    q[..., 0] = 1.5
+    k, v = (torch.randn(B, Hkv, cap, D, device="cuda", generator=g).to(dtype) for _ in range(2))
+    k[::2, :, 128:900, 0] = float("-inf")
+    lens = torch.full((B,), cap, dtype=torch.int32, device="cuda")
+    lens[::4] = 700  # ends among them
+    if page:
+        per = cap // page
+        table = torch.arange(B * per, device="cuda", dtype=torch.int32).view(B, per)
+        kp, vp = (t.unflatten(2, (per, page)).transpose(1, 2).flatten(0, 1).contiguous() for t in (k, v))
+        o, lse = F.decode_attention_paged(q, kp, vp, table, lens, chunk=chunk)
+    else:
+        o, lse = F.decode_attention(q, k, v, lens, chunk=chunk)
+    torch.cuda.synchronize()
+    for b in (0, 1, 2, 3, B - 2, B - 1):
+        at = [t for t in range(int(lens[b])) if b % 2 or not 128 <= t < 900]
+        ro, rl = orc.sdpa_fwd(host(q[b:b + 1]), host(k[b:b + 1, :, at]), host(v[b:b + 1, :, at]), enable_gqa=True)
+        assert max_abs(host(o[b:b + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[b:b + 1]), rl[:, :, 0]) <= LSE_TOL
