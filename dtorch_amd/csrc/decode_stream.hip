@@ -431,6 +431,8 @@ bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hi
 bool decode_stream_fits(const DecodeParams& p, int32_t dtype, size_t ws_bytes, hipStream_t stream) {
     if ((dtype != DTATTN_BF16 && dtype != DTATTN_FP16) || p.d_real != kStreamD || p.group > kStreamHeads) return false;
     if (p.block_table != nullptr && (p.kspan == 0 || p.page_shift < 4)) return false;
+    // 16-byte loads straight into LDS and 8-byte stores (the entry points check strides, not pointers)
+    if (((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.k) | reinterpret_cast<uintptr_t>(p.v)) & 15u) != 0) return false;
     if ((reinterpret_cast<uintptr_t>(p.o) & 7u) != 0 || p.os_b % 4 != 0 || p.os_h % 4 != 0) return false;
     if (p.qs_h < 0 || p.qs_h * p.group >= (1 << 28) || p.ks_s < 0 || p.vs_s < 0) return false;
     if (!decode_stream_pays(p.B, p.Hkv, p.S_max, p.group, stream)) return false;

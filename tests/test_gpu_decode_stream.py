@@ -124,3 +124,31 @@ def test_parts_whose_scores_are_all_minus_infinity(page, chunk):
         at = [t for t in range(int(lens[b])) if b % 2 or not 128 <= t < 900]
         ro, rl = orc.sdpa_fwd(host(q[b:b + 1]), host(k[b:b + 1, :, at]), host(v[b:b + 1, :, at]), enable_gqa=True)
         assert max_abs(host(o[b:b + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[b:b + 1]), rl[:, :, 0]) <= LSE_TOL
+
+
+@pytest.mark.parametrize("which", ["q", "o"])
+def test_pointers_off_their_alignment_keep_the_split_form(which):
+    """The C ABI checks strides, not pointers: a query or output 4 elements into a buffer of a call large enough for the
+    streaming form takes the splits that chunk 0 picks beside it, bit for bit."""
+    import ctypes
+    from tests.test_zz_no_alloc import BF16, _args, _case
+    from tests.test_zz_no_alloc import _lib as bound
+    lib = bound()
+    B, S = 70, 1024
+    q, k, v, lengths = _case(B, 8, 2, S, 128, torch.bfloat16, B)
+    lengths.fill_(S - 3)
+
+    def moved(t, by):
+        return torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")[by:by + t.numel()].view(t.shape)
+
+    q = moved(q, 4 if which == "q" else 0).copy_(q)
+    outs = []
+    for chunk in (0, 384):
+        o, lse = moved(q, 2 if which == "o" else 0), torch.empty(B, 8, device="cuda")
+        ws = torch.empty(lib.dtattn_decode_workspace_size(B, 8, S, 128, 0), dtype=torch.uint8, device="cuda")
+        a = _args(q, k, v, lengths, o, lse, BF16, chunk, ws)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert lib.dtattn_decode_splitkv(ctypes.byref(a), stream) == 0, lib.dtattn_last_error()
+        outs.append((o, lse))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
