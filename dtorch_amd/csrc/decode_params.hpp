@@ -34,8 +34,10 @@ struct DecodeParams {
     uint32_t q_and, q_xor;  // applied to q's words at load, as in ScalePlan
 };
 
+// CUs of the stream's device (0: unknown).
+int stream_cus(hipStream_t stream);
 // Whether a 16-bit call at head dim 128 is large enough for the streaming form.
-bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hipStream_t stream);
+bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, bool paged, hipStream_t stream);
 // The streaming form (decode_stream.hip): whether a call on the current device takes it (its partials fit `ws_bytes`),
 // and its two launches.
 bool decode_stream_fits(const DecodeParams& p, int32_t dtype, size_t ws_bytes, hipStream_t stream);

@@ -45,16 +45,34 @@ size_t decode_ws_parts(int64_t B, int64_t Hq, int64_t S_max, int64_t D_real, int
 // 1-128, contexts 2K-128K, 4 heads per workgroup: 384 was 1-8% faster than 256 at D = 64 and 128
 // everywhere except one 8K sequence (-1 to -2%); 256 had been best or within 2% of 128 and 512.
 //
-// 16-bit calls at head dim 128 in groups of 3 to 8 heads that are too small for the streaming form take 128 as well: their
-// grids leave CUs idle, and a third of the bytes per workgroup ends sooner than the merge of three times the partials
-// costs (32 heads over 8, per call: 1x500 12.0 -> 8.2 us, 1x4000 12.4 -> 9.3, 4x1000 13.2 -> 8.9, 16x500 14.5 -> 11.9; 64
-// over 8: 1x4000 13.3 -> 12.5; 28 over 4: 1x1000 8.2 -> 6.9, 1x8000 15.4 -> 15.7, the one size it loses).  Where the
-// streaming form is out for another reason (a pool past 4 GB), 384 stays above that bound.
-static int32_t auto_chunk(int64_t B, int64_t Hq, int64_t Hkv, int64_t S_max, int64_t D, int64_t esz, size_t ws_bytes,
-                          hipStream_t stream) {
+// 16-bit calls at head dim 128 in groups of 3 to 8 heads that are too small for the streaming form may take 128 as well: their
+// grids leave CUs idle, and a third of the bytes per workgroup ends sooner, until the merge of three times the partials
+// (or a second and third round of workgroups) costs more.  us a call at 384 / 128 tokens:
+//   up to 128 tokens of capacity: one split either way, no merge (1x128 groups of 4 8.9 / 5.2, of 3 4.8 / 3.2)
+//   up to 384: 384 is one split, without the merge launch (groups of 3 1x256 4.7 / 6.4, 16x384 8.1 / 10.1; of 6 1x256 5.8 / 7.1); in
+//     groups of 4 and 8 its workgroups of 4 heads load long enough for 128 to win while those fit the CUs once (4: 1x256
+//     8.9 / 8.4, 16x256 10.1 / 9.6, 16x384 10.5 / 11.3; 8: 4x384 9.9 / 8.9, 16x256 10.0 / 12.1)
+//   groups of 4 above that: but for one sequence of more than 64 partials a head, whose merge is the chain (1x4000 12.5 / 9.4,
+//     1x8032 14.7 / 13.6, 1x10080 15.8 / 16.6, 1x12128 16.0 / 18.0; 2x5984 15.5 / 16.0 and half full 12.2 / 11.2, 4x2912 15.1 / 15.3,
+//     16x880 20.4 / 16.8); of 8 while the workgroups fit twice (4x944 13.1 / 11.4, 2x2400 13.6 / 14.7, 1x5984 14.4 / 16.5)
+//   groups of 3, 5 and 7 (workgroups of one head, few bytes each): up to 2560 tokens (5: 1x1008 8.9 / 7.5, 2x2560 13.2 / 12.8,
+//     1x6144 14.5 / 15.2; 7: 4x2000 15.1 / 14.0, 1x3072 9.1 / 9.7, 1x8000 16.4 / 16.4); of 6 up to 1536 (8x896 16.8 / 13.8, 4x1536 13.5 /
+//     13.6, 2x3072 12.7 / 13.5)
+// Where the streaming form is out for another reason (a pool past 4 GB), 384 stays.
+static bool small_splits(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hipStream_t stream) {
+    if (S_max <= 128) return true;
+    if (group % 4 != 0) return S_max > 384 && S_max <= (group % 2 != 0 ? 2560 : 1536);
+    const int64_t workgroups = B * Hkv * (group / 4) * ((S_max + 127) / 128), cus = stream_cus(stream);
+    if (S_max <= 384) return workgroups <= cus;
+    return group == 4 ? B > 1 || S_max <= 8192 : workgroups <= 2 * cus;
+}
+
+static int32_t auto_chunk(int64_t B, int64_t Hq, int64_t Hkv, int64_t S_max, int64_t D, int64_t esz, bool paged,
+                          size_t ws_bytes, hipStream_t stream) {
     const int64_t group = Hq / Hkv;
     if (group % 8 == 0 && Hkv % 8 != 0) return 128;
-    if (esz == 2 && D == 128 && group >= 3 && group <= 8 && !decode_stream_pays(B, Hkv, S_max, group, stream) &&
+    if (esz == 2 && D == 128 && group >= 3 && group <= 8 && !decode_stream_pays(B, Hkv, S_max, group, paged, stream) &&
+        small_splits(B, Hkv, S_max, group, stream) &&
         decode_ws_parts(B, Hq, S_max, D, 128, nullptr) <= ws_bytes)  // a workspace sized for 384 keeps 384
         return 128;
     return esz == 2 ? 384 : 256;
@@ -548,7 +566,7 @@ static int decode_splitkv_run(const dtattn_decode_args* a, void* ws, size_t ws_b
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, a->S_max, a->D, esz, noalloc ? kScratchBytes : ws_bytes, stream);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, a->S_max, a->D, esz, false, noalloc ? kScratchBytes : ws_bytes, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode: chunk %d must be 128, 256, 384 or 512", chunk);
     // chunk rows are addressed with 32-bit byte offsets
@@ -653,7 +671,7 @@ extern "C" int dtattn_decode_paged(const dtattn_decode_paged_args* a, void* stre
     if (a->dtype != DTATTN_BF16 && a->dtype != DTATTN_FP16 && a->dtype != DTATTN_FP32)
         return fail(DTATTN_ERR_UNSUPPORTED, "decode_paged: dtype %d not supported (bf16, fp16, fp32)", a->dtype);
     const int64_t esz = a->dtype == DTATTN_FP32 ? 4 : 2;
-    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, S_max, a->D, esz, a->workspace_bytes, stream);
+    const int32_t chunk = a->chunk > 0 ? a->chunk : auto_chunk(a->B, a->Hq, a->Hkv, S_max, a->D, esz, true, a->workspace_bytes, stream);
     if (chunk != 128 && chunk != 256 && chunk != 384 && chunk != 512)
         return fail(DTATTN_ERR_INVALID_ARGUMENT, "decode_paged: chunk %d must be 128, 256, 384 or 512", chunk);
     if (a->q == nullptr || a->k_pages == nullptr || a->v_pages == nullptr || a->block_table == nullptr ||

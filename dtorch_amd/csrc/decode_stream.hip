@@ -404,7 +404,7 @@ __global__ void __launch_bounds__(256) decode_stream_merge_kernel(const DecodePa
     if (p.lse != nullptr && lane == 0) p.lse[b * p.lses_b + hq] = mx + __logf(sum);
 }
 
-static int stream_cus(hipStream_t stream) {
+int stream_cus(hipStream_t stream) {
     int dev = 0;
     dtattn_device_peaks pk;
     if ((stream == nullptr ? hipGetDevice(&dev) : hipStreamGetDevice(stream, &dev)) != hipSuccess) return 0;
@@ -417,13 +417,26 @@ static int stream_shares(const DecodeParams& p, hipStream_t stream) {
     return (int)std::min<int64_t>(4 * (int64_t)stream_cus(stream), (int64_t)p.B * p.Hkv * ((p.S_max + 127) / 128) / 2);
 }
 
-// Units per CU from which it is faster, by the capacity (the host does not know the lengths).  Its fixed cost is about 2 us
-// above the split form's; that form reads a chunk twice for 8 heads and 7 times for 7, and keeps up longest where
-// every head reads its own cache (1: 16x1000 44.0 against 46.9 us, 16x2000 86.9 against 84.6; 4: 16x500 15.1 against
-// 16.4, 16x1000 21.7 against 17.9; 8: 4x1000 14.4 against 16.3, 16x500 19.7 against 16.5;
-// 7: 8x1000 13.4 against 15.9).
-bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, hipStream_t stream) {
-    const int64_t per_cu = group >= 5 ? 6 : group >= 3 ? 15 : 124;
+// Units per CU from which it is faster, by the capacity (the host does not know the lengths).  Its fixed cost is about 3 us
+// above the split form's, which reads a chunk twice for 8 heads, three times for 6 and 3, and 5 and 7 times for 5 and 7, and
+// keeps up longest where every head reads its own cache.  A line is where the form wins on full caches and loses little
+// on half-full ones.  us, 384-token splits (the form's own alternative above 2560 tokens) / streaming, full and half full:
+//   1: contiguous 16x8192 340 / 339 and 16x512 in 8192 30 / 33, 64x512 91 / 101: never; pages of 16 tokens 64x512 99 / 86,
+//      64x2048 365 / 329, 16x2048 mixed 53 / 49
+//   2: 64x2048 94 / 88, 16x8192 mixed 53 / 50 (128 units); 16x2048 26.7 / 27.3 (32)
+//   3: 4x3072 16.8 / 17.1 and 11.7 / 12.3 (12 units); 4x3840 20.9 / 17.4 and 11.8 / 12.6, 16x960 21.6 / 17.8 and 14.1 / 13.0 (15)
+//   4: 4x2912 15.1 / 17.3 (11); 4x3680 20.9 / 17.6 and 13.7 / 13.2 (14); up to 384 tokens 64x384 19.8 / 23.3 (24), 3: 64x256
+//      19.8 / 23.4 (16): never
+//   5: 4x2048 16.9 / 16.3 and 9.8 / 12.0 (8); 4x3072 22.4 / 17.3 and 13.1 / 12.4 (12);  6: 4x2048 16.6 / 16.2 and 11.4 / 12.0 (8);
+//      4x3072 20.0 / 17.3 and 12.2 / 12.5 (12)
+//   7: 4x2048 14.9 / 16.2 (4); 4x3072 20.1 / 16.1 and 12.3 / 11.9, 64x192 20.1 / 11.7 (6)
+//   8: 4x1536 14.2 / 16.2 (6); 2x3936 19.8 / 16.8 and 12.4 / 12.8, 16x448 19.1 / 15.4 (7)
+// Lengths far below the capacity (a sixteenth and less) cost it up to 3.5 us (7: 1x2048 in 32768 8.3 / 10.0; 3: 4x256 in 4096
+// 6.3 / 9.6), in groups of 4 and 8 nothing (4: 1x2048 in 32768 11.9 / 9.9).
+bool decode_stream_pays(int64_t B, int64_t Hkv, int64_t S_max, int64_t group, bool paged, hipStream_t stream) {
+    if (group > kStreamHeads || (group == 1 && !paged)) return false;
+    if (group <= 4 && S_max <= 384) return false;  // one split per sequence and no merge
+    const int64_t per_cu = group == 8 ? 7 : group == 7 ? 6 : group >= 5 ? 12 : group >= 3 ? 15 : 124;
     const int cus = stream_cus(stream);
     return cus > 0 && B * Hkv * ((S_max + kUnit - 1) / kUnit) >= per_cu * cus;
 }
@@ -435,7 +448,7 @@ bool decode_stream_fits(const DecodeParams& p, int32_t dtype, size_t ws_bytes, h
     if (((reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.k) | reinterpret_cast<uintptr_t>(p.v)) & 15u) != 0) return false;
     if ((reinterpret_cast<uintptr_t>(p.o) & 7u) != 0 || p.os_b % 4 != 0 || p.os_h % 4 != 0) return false;
     if (p.qs_h < 0 || p.qs_h * p.group >= (1 << 28) || p.ks_s < 0 || p.vs_s < 0) return false;
-    if (!decode_stream_pays(p.B, p.Hkv, p.S_max, p.group, stream)) return false;
+    if (!decode_stream_pays(p.B, p.Hkv, p.S_max, p.group, p.block_table != nullptr, stream)) return false;
     if ((int64_t)p.B * p.Hkv * ((p.S_max + kUnit - 1) / kUnit) >= ((int64_t)1 << 31)) return false;
     const int n = stream_shares(p, stream);
     return n > 0 && (size_t)(2 * n) * p.group * (kStreamD + 1) * sizeof(float) <= ws_bytes;

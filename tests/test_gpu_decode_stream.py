@@ -152,3 +152,74 @@ def test_pointers_off_their_alignment_keep_the_split_form(which):
         outs.append((o, lse))
     torch.cuda.synchronize()
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+# units of 32 tokens per CU from which a group of query heads takes the streaming form (1: paged caches only)
+LINE = {1: 124, 2: 124, 3: 15, 4: 15, 5: 12, 6: 12, 7: 6, 8: 7}
+
+
+@pytest.mark.parametrize("group", sorted(LINE))
+@pytest.mark.parametrize("page", [0, 16])
+@pytest.mark.parametrize("B", [2, 67])  # merged by four waves a head, and by one
+def test_every_group_on_both_sides_of_its_line(group, page, B):
+    """The streaming form from its line on, and the splits that chunk 0 picks just below it, against splits of 256 and
+    the oracle.  Forms differ in the last bits of some LSE, so a chunk 0 that matches neither split length ran the
+    streaming kernel."""
+    import dtorch_amd.nn.functional as F
+    D, dtype = 128, torch.bfloat16
+    Hkv = 8 if group <= 2 else 4
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    units = LINE[group] * cus // (B * Hkv) + 1  # a sequence
+    g = torch.Generator(device="cuda").manual_seed(group + page)
+    q = torch.randn(B, Hkv * group, 1, D, device="cuda", generator=g).to(dtype)
+    for u in (units, units - 2):
+        cap = 32 * u
+        streams = B * Hkv * u >= LINE[group] * cus and (group > 1 or page > 0)
+        assert streams == (u == units and (group > 1 or page > 0))
+        k, v = (torch.randn(B, Hkv, cap, D, device="cuda", generator=g).to(dtype) for _ in range(2))
+        lens = torch.randint(0, cap + 1, (B,), device="cuda", generator=g, dtype=torch.int32)
+        lens[0], lens[B - 1] = cap - 1, cap
+        if page:
+            per = cap // page
+            table = torch.randperm(B * per, device="cuda", generator=g).view(B, per)
+            pages = []
+            for t in (k, v):
+                pool = torch.empty(B * per, Hkv, page, D, dtype=dtype, device="cuda")
+                pool[table.flatten()] = t.unflatten(2, (per, page)).transpose(1, 2).flatten(0, 1)
+                pages.append(pool)
+            run = lambda chunk: F.decode_attention_paged(q, *pages, table.to(torch.int32), lens, chunk=chunk)
+        else:
+            run = lambda chunk: F.decode_attention(q, k, v, lens, chunk=chunk)
+        o, lse = run(0)
+        os_, ls = run(256)
+        same = [torch.equal(lse, run(c)[1]) for c in (128, 384)]
+        torch.cuda.synchronize()
+        assert any(same) != streams
+        assert max_abs(host(o), host(os_)) <= O_TOL_BF16
+        fin = ~torch.isneginf(ls)
+        assert torch.equal(fin, ~torch.isneginf(lse)) and lse_rel(host(lse[fin]), host(ls[fin])) <= 1e-5
+        for b in (0, B - 1):
+            n = int(lens[b])
+            ro, rl = orc.sdpa_fwd(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), enable_gqa=True)
+            assert max_abs(host(o[b:b + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[b:b + 1]), rl[:, :, 0]) <= LSE_TOL
+
+
+@pytest.mark.parametrize("group", [3, 4, 5, 6, 8])
+@pytest.mark.parametrize("B,cap", [(1, 128), (1, 129), (1, 384), (1, 385), (20, 384), (1, 1536), (1, 1537), (2, 2560), (2, 2561), (1, 3073),
+                                   (1, 8193), (9, 600)])
+def test_split_lengths_of_smaller_calls(group, B, cap):
+    """The bounds between splits of 128 and of 384 tokens (one split, a merge or none) against splits of 256."""
+    import dtorch_amd.nn.functional as F
+    Hkv, D, dtype = 8, 128, torch.float16
+    g = torch.Generator(device="cuda").manual_seed(group + cap)
+    q = torch.randn(B, Hkv * group, 1, D, device="cuda", generator=g).to(dtype)
+    k, v = (torch.randn(B, Hkv, cap, D, device="cuda", generator=g).to(dtype) for _ in range(2))
+    for n in (cap, cap - 1, 1, 0):
+        lens = torch.full((B,), n, dtype=torch.int32, device="cuda")
+        o, lse = F.decode_attention(q, k, v, lens)
+        ro, rl = F.decode_attention(q, k, v, lens, chunk=256)
+        torch.cuda.synchronize()
+        if n == 0:
+            assert not o.any() and torch.isneginf(lse).all()
+            continue
+        assert max_abs(host(o), host(ro)) <= O_TOL_BF16 and lse_rel(host(lse), host(rl)) <= 1e-5
