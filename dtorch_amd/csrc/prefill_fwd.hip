@@ -49,7 +49,8 @@ __device__ __forceinline__ int kswz(int r) {
 // p.qk_ch and V chunks past p.v_ch load as zeros, and O chunks past p.v_ch are not stored.
 // KG: key groups.  KG * 4 waves share the 128 query rows, group g takes key tiles g, g + KG, ... through its own LDS
 // buffers, and the groups' (O, max, sum) are merged in fp32 through LDS: for grids that leave CUs idle otherwise.
-template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG = 1>
+// SUMC: the row max only where the sums of P ask for it (below).
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG, bool SUMC>
 __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel(const PrefillParams p) {
     constexpr int NW = 4;
     constexpr int BN = 64;
@@ -111,12 +112,12 @@ __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel
 #pragma unroll
         for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
     float mrow = kNegInf, lrow = 0.f;
-    // The VALU work of the softmax, not the MFMAs, bounds head dim 64, and the row max is a tenth of it.  Non-causal
-    // kernels without a mask compute it only when it has to move: a tile is exponentiated with the max so far, and only
+    // The VALU work of the softmax, not the MFMAs, bounds head dim 64, and the row max is a tenth of it.  SUMC (non-causal
+    // kernels without a mask) computes it only when it has to move: a tile is exponentiated with the max so far, and only
     // if some lane's sum of its 32 P then exceeds 2^8 (no sum up to it holds a P above the bound that the rescale rule
     // keeps) are the row max, the rescale and the exponentials done over; also while a row has no max yet.  2x24x4429
-    // fp16 304 -> 286 us, 4x24x2304 161 -> 157; with the causal or masked kernels' registers it cost 2-6%.
-    constexpr bool kSumCheck = D == 64 && !CAUSAL && MASKED == kMaskNone;
+    // fp16 286 -> 271 us; with the causal or masked kernels' registers it cost 2-6%.  sum_check_pays() has the grids.
+    static_assert(!SUMC || (D == 64 && !CAUSAL && MASKED == kMaskNone), "the kernels of the form");
     constexpr float kSumLimit = 256.f;  // 2^kRescaleThreshold
     bool fresh = true;
 
@@ -293,7 +294,7 @@ __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel
         // Wave priority: raised over the exponential/PV block of the non-causal kernel only.  Measured
         // A/B on one MI355X: MMDiT 1x24x4608 +4.5% against raising it over both blocks; the causal
         // kernels ran 1-3% faster with no raise at all.
-        if constexpr (kSumCheck) {
+        if constexpr (SUMC) {
             float ls = 0.f;
             bool done = false;
             if (!fresh) {
@@ -452,7 +453,7 @@ __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel
 
 // ------------------------------------------------------------------------------------------------
 
-template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG = 1>
+template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG = 1, bool SUMC = false>
 static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     constexpr int BM = 4 * QT * 32;
     PrefillParams p = prm;
@@ -460,8 +461,29 @@ static int launch_prefill(const PrefillParams& prm, hipStream_t stream) {
     const int64_t grid = (int64_t)p.n_qblocks * p.B * p.Hq;
     if (grid == 0) return DTATTN_OK;
     if (grid > 0x7fffffff) return fail(DTATTN_ERR_UNSUPPORTED, "prefill grid too large (%lld blocks)", (long long)grid);
-    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, QT, CAUSAL, MASKED, PAD, KG>), dim3((unsigned)grid), dim3(256 * KG), 0, stream, p);
+    hipLaunchKernelGGL((prefill_fwd_kernel<T, D, QT, CAUSAL, MASKED, PAD, KG, SUMC>), dim3((unsigned)grid), dim3(256 * KG), 0, stream, p);
     return check_launch("prefill_fwd_kernel");
+}
+
+static int stream_device(hipStream_t stream, int* dev) {
+    return (stream == nullptr ? hipGetDevice(dev) : hipStreamGetDevice(stream, dev)) == hipSuccess ? DTATTN_OK
+                                                                                               : DTATTN_ERR_DEVICE;
+}
+
+// Whether a head-dim-64 call without mask or causal rule takes the form that checks the sums of P.  With r workgroups of
+// 128 rows per CU (three fit at once), times with the row max first over times with the check, bf16 / fp16:
+//   r up to 2: 1.03-1.37 from 512 keys on, 0.94-1.00 at 77 to 256 keys
+//   2 < r <= 3: 0.96-0.99 at r = 2.25, 0.96-1.00 at 2.5, 0.98-1.01 at 2.75 and 3, at any number of keys
+//   3 < r <= 4: 1.02-1.10 at 3.25; at 3.75 and 4 1.01-1.07 up to 256 keys, 0.95-0.97 at 512 and 768, 0.96-1.01 above
+//   r above 4: 1.00-1.08 (one 0.97)
+static bool sum_check_pays(const PrefillParams& p, hipStream_t stream) {
+    int dev = 0;
+    dtattn_device_peaks pk;
+    if (stream_device(stream, &dev) != DTATTN_OK || dtattn_get_device_peaks(dev, &pk) != DTATTN_OK) return true;
+    const int64_t grid = ((int64_t)p.Sq + 127) / 128 * p.B * p.Hq, cus = pk.cu_count;
+    if (grid > 4 * cus) return true;
+    if (grid > 3 * cus) return 8 * grid <= 27 * cus || p.Sk <= 256;
+    return grid <= 2 * cus && p.Sk > 256;
 }
 
 template <typename T, int MASKED, bool PAD>
@@ -472,13 +494,15 @@ static int dispatch_prefill_m(const PrefillParams& p, int D, bool causal, int kg
                           : launch_prefill<T, 128, 1, false, MASKED, PAD, 2>(p, stream);
         if (kg > 1 && D == 64)
             return causal ? launch_prefill<T, 64, 1, true, MASKED, PAD, 2>(p, stream)
-                          : launch_prefill<T, 64, 1, false, MASKED, PAD, 2>(p, stream);
+                          : launch_prefill<T, 64, 1, false, MASKED, PAD, 2, true>(p, stream);
     }
     if (D == 128) {
         return causal ? launch_prefill<T, 128, 1, true, MASKED, PAD>(p, stream)
                       : launch_prefill<T, 128, 1, false, MASKED, PAD>(p, stream);
     }
     if (D == 64) {
+        if constexpr (MASKED == kMaskNone)
+            if (!causal && sum_check_pays(p, stream)) return launch_prefill<T, 64, 1, false, MASKED, PAD, 1, true>(p, stream);
         return causal ? launch_prefill<T, 64, 1, true, MASKED, PAD>(p, stream)
                       : launch_prefill<T, 64, 1, false, MASKED, PAD>(p, stream);
     }
@@ -578,11 +602,6 @@ static MaskSpans mask_spans_plan(const dtattn_prefill_args* a, const dtattn_mask
         m.bytes = m.rows + (size_t)a->B * m.pitch * sizeof(float);
     }
     return m;
-}
-
-static int stream_device(hipStream_t stream, int* dev) {
-    return (stream == nullptr ? hipGetDevice(dev) : hipStreamGetDevice(stream, dev)) == hipSuccess ? DTATTN_OK
-                                                                                               : DTATTN_ERR_DEVICE;
 }
 
 // Key groups of prefill_fwd_kernel for a call without mask or padding, or 0: the grid is large enough for the kernels

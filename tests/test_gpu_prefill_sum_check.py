@@ -29,3 +29,23 @@ def test_rising_scores(Sq, Sk, step, dtype):
     o, lse = F.scaled_dot_product_attention_with_lse(tq, tk, tv)
     torch.cuda.synchronize()
     assert max_abs(host(o), ro) <= O_TOL_BF16 and lse_rel(host(lse), rl) <= LSE_TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,Sk", [(0.9, 300), (1.5, 256), (1.5, 257), (2.5, 320), (3.2, 600), (3.8, 600), (3.8, 200), (4.5, 129)])
+def test_forms_by_grid(r, Sk, dtype):
+    """Grids of r workgroups per CU, on each side of the lines between the form that checks the sums and the one that
+    takes the row max first: the scores of the test above (steps of 4), some heads against the oracle."""
+    import dtorch_amd.nn.functional as F
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.default_rng(Sk + int(10 * r))
+    Sq, H = 130, int(r * cus) // 2  # two workgroups a head
+    q, k, v = randn(rng, (1, H, Sq, 64)), 0.3 * randn(rng, (1, 1, Sk, 64)), randn(rng, (1, 1, Sk, 64))
+    q[..., 0] = np.resize([1.0, -1.0, 0.0], Sq)
+    k[..., 0] = (np.arange(Sk) // 64) * 4.0 * np.log(2.0) * 8.0
+    tq, tk, tv = (torch.from_numpy(x).to(dtype).cuda() for x in (q, k, v))
+    o, lse = F.scaled_dot_product_attention_with_lse(tq, tk, tv, enable_gqa=True)
+    torch.cuda.synchronize()
+    for h in (0, H // 2, H - 1):
+        ro, rl = orc.sdpa_fwd(*(host(t).astype(np.float64) for t in (tq[:, h:h + 1], tk, tv)))
+        assert max_abs(host(o[:, h:h + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[:, h:h + 1]), rl) <= LSE_TOL
