@@ -608,7 +608,9 @@ static MaskSpans mask_spans_plan(const dtattn_prefill_args* a, const dtattn_mask
 // with 64 rows per wave (head dim 128).  A workgroup ends no sooner than its own key tiles, and a 64-row wave takes
 // 1.35 us a tile against 0.95 us here, so up to two workgroups per CU 128-row blocks of one head end first (causal
 // 1x32/8x512 18.0 -> 13.8 us, 2x32/8x777 23.1 -> 20.4, 4x32/8x512 18.3 -> 15.8; 16x32/8x128 not causal 11.8 -> 9.5); a
-// non-causal grid of long rows is as good on the 64-row kernel already (1x32/8x1500 42.6 against 40.6).  Two key groups
+// non-causal grid of long rows is as good on the 64-row kernel already (1x32/8x1500 42.6 against 40.6; two workgroups per CU,
+// 64-row time over this one's at 640, 896 and 1024 keys: 1.10, 1.06, 1.04 for 16 kv heads, 1.05, 1.00, 0.97 where the 64-row
+// kernel shares a kv head's tiles among 4 query heads).  Two key groups
 // halve the chain of tiles, for 128 KB of LDS at head dim 128 and a merge worth 1-2 us: from 8 tiles on, on grids of one
 // workgroup per CU (causal 1x32/8x1024 22.3 -> 20.9, 777 18.2 -> 16.7, 400 11.9 both; D = 64 1x12x1024 15.8 -> 13.4) and
 // on causal ones of two where the second round is the short blocks of many (1x32/8x1500 32.0 -> 28.8, D = 64 1x12x4096
@@ -624,7 +626,7 @@ static int key_groups(const PrefillParams& p, int D, bool causal, hipStream_t st
     if (grid <= pk.cu_count) return tiles >= 8 ? 2 : 1;
     if (grid <= 2 * pk.cu_count) {
         if (causal) return tiles >= 8 && blocks >= 12 ? 2 : 1;
-        if (tiles <= 16) return 1;
+        if (tiles <= (p.group >= 4 && p.group % 4 == 0 ? 13 : 16)) return 1;
     }
     return D == 128 ? 0 : 1;
 }
