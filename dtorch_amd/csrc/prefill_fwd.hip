@@ -47,11 +47,12 @@ __device__ __forceinline__ int kswz(int r) {
 
 // PAD: the real head dims are below D (any multiple of 8, Dv may differ from D); Q/K chunks past
 // p.qk_ch and V chunks past p.v_ch load as zeros, and O chunks past p.v_ch are not stored.
-// KG: key groups.  KG * 4 waves share the 128 query rows, group g takes key tiles g, g + KG, ... through its own LDS
-// buffers, and the groups' (O, max, sum) are merged in fp32 through LDS: for grids that leave CUs idle otherwise.
+// KG: key groups, 1 or 2.  KG * 4 waves share the 128 query rows, group g takes key tiles g, g + KG, ... through its own
+// LDS buffers, and the groups' (O, max, sum) are merged in fp32 through LDS: for grids that leave CUs idle otherwise.
 // SUMC: the row max only where the sums of P ask for it (below).
 template <typename T, int D, int QT, bool CAUSAL, int MASKED, bool PAD, int KG, bool SUMC>
-__global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel(const PrefillParams p) {
+__global__ void __launch_bounds__(256 * KG, 2) prefill_fwd_kernel(const PrefillParams p) {
+    static_assert(KG == 1 || KG == 2, "the merge holds one more group");
     constexpr int NW = 4;
     constexpr int BN = 64;
     constexpr int BM = NW * 32;
@@ -374,38 +375,29 @@ __global__ void __launch_bounds__(256 * KG, KG <= 2 ? 2 : KG) prefill_fwd_kernel
         if (t + KG < nt) tile(Kb, Vb, Ka, Va, t + KG + kg);
     }
     if constexpr (KG > 1) {
-        // Groups past the first leave their 16 DT accumulators, max and sum per lane in LDS; the first merges them.
+        // The second group leaves its 16 DT accumulators, max and sum per lane in LDS; the first merges them.
         __syncthreads();
-        auto part = [&](int g) {  // [16 DT][64 lanes] of this wave's rows from group g: KG slots per buffer
-            const int s = (g - 1) * NW + wave;
-            T* const buf = s < KG ? Ka_ : s < 2 * KG ? Kb_ : Va_;
-            return reinterpret_cast<float*>(buf + (s % KG) * BN * D);
-        };
-        float* const ml = reinterpret_cast<float*>(Vb_);
+        float* const part = reinterpret_cast<float*>((wave < 2 ? Ka_ : Kb_) + (wave & 1) * BN * D);  // [16 DT][64 lanes]
+        float* const ml = reinterpret_cast<float*>(Vb_) + wave * 128;
         if (kg > 0) {
-            float* const dst = part(kg);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) dst[(16 * dt + i) * 64 + lane] = oacc[dt][i];
-            ml[((kg * NW + wave) * 2 + 0) * 64 + lane] = mrow;
-            ml[((kg * NW + wave) * 2 + 1) * 64 + lane] = lrow;
+                for (int i = 0; i < 16; ++i) part[(16 * dt + i) * 64 + lane] = oacc[dt][i];
+            ml[lane] = mrow;
+            ml[64 + lane] = lrow;
         }
         __syncthreads();
         if (kg == 0) {
+            const float mg = ml[lane], lg = ml[64 + lane];
+            const float mm = fmaxf(mrow, mg), mb = mm == kNegInf ? 0.f : mm;  // -inf: no visible key, weight 0
+            const float a0 = fast_exp2(mrow - mb), ag = fast_exp2(mg - mb);
+            mrow = mm;
+            lrow = lrow * a0 + lg * ag;
 #pragma unroll
-            for (int g = 1; g < KG; ++g) {
-                const float* const src = part(g);
-                const float mg = ml[((g * NW + wave) * 2 + 0) * 64 + lane], lg = ml[((g * NW + wave) * 2 + 1) * 64 + lane];
-                const float mm = fmaxf(mrow, mg), mb = mm == kNegInf ? 0.f : mm;  // -inf: no visible key, weight 0
-                const float a0 = fast_exp2(mrow - mb), ag = fast_exp2(mg - mb);
-                mrow = mm;
-                lrow = lrow * a0 + lg * ag;
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a0 + src[(16 * dt + i) * 64 + lane] * ag;
-            }
+                for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * a0 + part[(16 * dt + i) * 64 + lane] * ag;
         }
     }
 
