@@ -427,15 +427,17 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) prefill_f32_ks_kernel(co
         }
         // every K(t) read has returned: K(t+4) may land
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (more) dma(Kt, kp, krow, p.ks_s, t + NW, p.qk_ch);
         if constexpr (MASKED != kMaskNone) {
+            // Before the tile loads: the compiler's waits for the mask values do not count those and would drain them.
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 float s0 = s[4 * g + 0], s1 = s[4 * g + 1], s2 = s[4 * g + 2], s3 = s[4 * g + 3];
                 mslab.add(mraw[g], p.inv_scale, s0, s1, s2, s3);
                 s[4 * g + 0] = s0, s[4 * g + 1] = s1, s[4 * g + 2] = s2, s[4 * g + 3] = s3;
             }
+            asm volatile("" : "+v"(s));  // keeps the adds, and so the waits, on this side of the loads
         }
+        if (more) dma(Kt, kp, krow, p.ks_s, t + NW, p.qk_ch);
         const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && (kbase + BN - 1 > q0 + p.delta));
         if (need_mask) {
             int lim = p.Sk - 1 - kbase;
@@ -841,6 +843,8 @@ static int launch_prefill_f32_wide(const PrefillParams& prm, hipStream_t stream)
 //            137.6 / 102.8, 4x16x2048 causal 296 / 288, 4x32x2048 causal 548 / 591
 //   D = 128: 1x8x512 causal 70.2 / 24.5, 2x16x1000 causal 135 / 101, not causal 137 / 159, 1x12x2048 causal
 //            263 / 135, 4x16x1000 causal 185 / 199
+//   with an fp32 mask, D = 64: 1x8x512 causal 42.6 / 13.4, 2x16x1000 causal 89.8 / 49.7, not causal 85.2 / 85.0, 4x16x1000 causal
+//            106 / 88.5; D = 128: 1x8x512 causal 85.0 / 24.2, 2x16x1000 causal 179 / 105
 static bool f32_key_split(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
     if (D != 64 && D != 128) return false;
     int dev = 0;
