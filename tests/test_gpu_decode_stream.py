@@ -223,3 +223,27 @@ def test_split_lengths_of_smaller_calls(group, B, cap):
             assert not o.any() and torch.isneginf(lse).all()
             continue
         assert max_abs(host(o), host(ro)) <= O_TOL_BF16 and lse_rel(host(lse), host(rl)) <= 1e-5
+
+
+def test_table_entries_outside_the_pool():
+    """Entries of the block table past a sequence's last page hold anything; one inside its length that is not a page of
+    the pool reads some page of it, and no other sequence notices."""
+    import dtorch_amd.nn.functional as F
+    B, Hq, Hkv, page, per, D = 70, 8, 2, 16, 64, 128
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randn(B, Hq, 1, D, device="cuda", generator=g).to(torch.bfloat16)
+    kp, vp = (torch.randn(B * per, Hkv, page, D, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    table = torch.randperm(B * per, device="cuda", generator=g).view(B, per).to(torch.int32)
+    lens = torch.randint(1, per * page + 1, (B,), device="cuda", generator=g, dtype=torch.int32)
+    lens[0] = 100
+    o, lse = F.decode_attention_paged(q, kp, vp, table, lens)
+    bad = table.clone()
+    past = torch.arange(per, device="cuda")[None] * page >= lens[:, None]
+    junk = torch.tensor([-1, -2 ** 31, B * per, 2 ** 31 - 1], dtype=torch.int32, device="cuda")
+    bad[past] = junk[torch.randint(0, 4, (int(past.sum()),), device="cuda", generator=g)]
+    o2, l2 = F.decode_attention_paged(q, kp, vp, bad, lens)
+    bad[0, 2] = 2 ** 31 - 1
+    o3, l3 = F.decode_attention_paged(q, kp, vp, bad, lens)
+    torch.cuda.synchronize()
+    assert torch.equal(o2, o) and torch.equal(l2, lse)
+    assert torch.equal(o3[1:], o[1:]) and torch.equal(l3[1:], lse[1:]) and o3.isfinite().all()
