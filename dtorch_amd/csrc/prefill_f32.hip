@@ -835,14 +835,18 @@ static int launch_prefill_f32_wide(const PrefillParams& prm, hipStream_t stream)
 }
 
 // Whether the key-split form is expected to beat the 128-row form, on a model in units of one 32-key tile of a
-// whole workgroup (about 2.1 us a CU at D = 64, 4.0 us at D = 128).  A grid cannot end before its longest item,
-// nor before its work is spread over the CUs; a causal grid, longest items first, ends about a quarter of its
-// longest item after that.  At full load the key-split form costs 6% (D = 64) or 30% (D = 128: one workgroup
-// per CU) more per tile.  Measured, 128-row against key-split form, us (B x H x S):
+// whole workgroup (about 2.1 us a CU at D = 64, 4.0 us at D = 128).  Not causal, all items are alike and a grid takes its
+// rounds of one per CU.  Causal, longest items first: up to one item per CU the longest; up to two, where a CU takes its
+// second as the first ends or runs both at once, the longest and the one that follows on its CU; beyond that the work
+// spread over the CUs and a tail of part of the longest.  At full load the key-split form costs 6% (D = 64) or 20%
+// (D = 128: one workgroup per CU) more per tile, and a tenth or half a tile per item, which at D = 128 nothing hides.  The
+// constants were fitted to 740 sizes (8 to 16 heads, batches of 1 to 8, 16 to 4096 tokens): in two of those for which the
+// model picks this form it is over 1.5% slower than the other (6% at 8x12x512 causal, D = 128).  Measured, 128-row against key-split form, us (B x H x S):
 //   D = 64:  1x8x512 causal 38.5 / 13.1, 2x16x1000 causal 72.9 / 46.7, not causal 71.8 / 71.9, 1x12x2048
 //            137.6 / 102.8, 4x16x2048 causal 296 / 288, 4x32x2048 causal 548 / 591
 //   D = 128: 1x8x512 causal 70.2 / 24.5, 2x16x1000 causal 135 / 101, not causal 137 / 159, 1x12x2048 causal
-//            263 / 135, 4x16x1000 causal 185 / 199
+//            263 / 135, 4x16x1000 causal 185 / 199, 8x16x200 causal 36.7 / 46.6, 8x12x777 causal 184 / 210, 8x16x384 not causal
+//            105 / 121, 2x8x3000 causal 488 / 342, 2x16x1536 causal 256 / 205
 //   with an fp32 mask, D = 64: 1x8x512 causal 42.6 / 13.4, 2x16x1000 causal 89.8 / 49.7, not causal 85.2 / 85.0, 4x16x1000 causal
 //            106 / 88.5; D = 128: 1x8x512 causal 85.0 / 24.2, 2x16x1000 causal 179 / 105
 static bool f32_key_split(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
@@ -852,32 +856,28 @@ static bool f32_key_split(const PrefillParams& p, int D, bool causal, hipStream_
     if ((stream == nullptr ? hipGetDevice(&dev) : hipStreamGetDevice(stream, &dev)) != hipSuccess ||
         dtattn_get_device_peaks(dev, &pk) != DTATTN_OK || pk.cu_count <= 0)
         return false;
-    const int64_t heads = (int64_t)p.B * p.Hq, blocks = ((int64_t)p.Sq + 127) / 128, cus = pk.cu_count;
-    if (heads * blocks > 8 * cus) return false;  // many rounds: the 128-row form (and a bound on the sums below)
-    const double e = D == 64 ? 1.06 : 1.3;
-    // tiles of the rows of block i (rows each), and their sum over the blocks
-    auto tiles = [&](int64_t i, int64_t rows) {
-        const int64_t lim = causal ? (i + 1) * rows + p.delta : p.Sk;
-        const int64_t kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
-        return (kend + 31) / 32;
+    const int64_t heads = (int64_t)p.B * p.Hq, cus = pk.cu_count;
+    if (heads * (((int64_t)p.Sq + 127) / 128) > 8 * cus) return false;  // many rounds: the 128-row form (and a bound on the sums below)
+    // items of `rows` rows whose key tiles `split` waves share; `over` tiles more per item, `tail` of the longest at the end;
+    // pairs: up to two items per CU end as the longest and its successor do
+    auto cost = [&](int64_t rows, int64_t split, double over, double tail, bool pairs) {
+        auto tiles = [&](int64_t i) {
+            const int64_t lim = causal ? (i + 1) * rows + p.delta : p.Sk;
+            const int64_t kend = lim < 0 ? 0 : (lim < p.Sk ? lim : p.Sk);
+            return ((kend + 31) / 32 + split - 1) / split;
+        };
+        const int64_t n = ((int64_t)p.Sq + rows - 1) / rows, items = heads * n;
+        const double longest = (double)tiles(n - 1) + over;  // causal: later rows see more keys
+        if (!causal) return (double)((items + cus - 1) / cus) * longest;
+        if (items <= cus) return longest;
+        if (pairs && items <= 2 * cus) return longest + (double)tiles(n - 1 - cus / heads) + over;
+        int64_t sum = 0;
+        for (int64_t i = 0; i < n; ++i) sum += tiles(i);
+        const double spread = ((double)(sum * heads) + over * (double)items) / (double)cus + tail * (longest - over);
+        return spread > longest ? spread : longest;
     };
-    int64_t sum = 0, sum_ks = 0, longest = 0, longest_ks = 0;
-    for (int64_t i = 0; i < blocks; ++i) {
-        const int64_t t = tiles(i, 128);
-        sum += t;
-        longest = t > longest ? t : longest;
-    }
-    for (int64_t i = 0; i * 32 < p.Sq; ++i) {
-        const int64_t t = (tiles(i, 32) + 3) / 4;
-        sum_ks += t;
-        longest_ks = t > longest_ks ? t : longest_ks;
-    }
-    auto cost = [&](int64_t total, int64_t chain, int64_t items) {
-        if (!causal) return (double)((items + cus - 1) / cus) * (double)chain;
-        const double spread = (double)(total * heads) / (double)cus + 0.25 * (double)chain;
-        return spread > (double)chain ? spread : (double)chain;
-    };
-    return e * cost(sum_ks, longest_ks, heads * (((int64_t)p.Sq + 31) / 32)) < cost(sum, longest, heads * blocks);
+    if (D == 64) return 1.06 * cost(32, 4, 0.1, 0.1, false) < cost(128, 1, 0.0, 0.2, true);
+    return 1.2 * cost(32, 4, 0.5, 0.1, true) < cost(128, 1, 0.0, 0.0, true);
 }
 
 template <int MASKED, bool PAD>

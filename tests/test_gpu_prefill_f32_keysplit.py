@@ -53,3 +53,21 @@ def test_key_split_against_128_row_form(Sq, Sk, D, Dv, causal, q_off, k_off, mas
     torch.cuda.synchronize()
     assert max_abs(host(o), ro) <= TOL and lse_rel(host(lse), rl) <= TOL
     assert max_abs(host(o[0]), host(ob[n - 1])) <= TOL and lse_rel(host(lse[0]), host(lb[n - 1])) <= TOL
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("r", [0.4, 0.9, 1.5, 2.5, 9])
+def test_forms_by_grid(r, D, causal):
+    """Grids of r 128-row items per CU, through every branch of the rule that picks a form: some heads against the oracle."""
+    import dtorch_amd.nn.functional as F
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.default_rng(int(10 * r) + D)
+    S, H = 200, int(r * cus) // 2  # two items a head
+    q, k, v = randn(rng, (1, H, S, D)), randn(rng, (1, 1, S + 40, D)), randn(rng, (1, 1, S + 40, D))
+    kw = dict(is_causal=causal, enable_gqa=True, q_offset=40)
+    o, lse = F.scaled_dot_product_attention_with_lse(*(torch.from_numpy(x).cuda() for x in (q, k, v)), **kw)
+    torch.cuda.synchronize()
+    for h in (0, H // 2, H - 1):
+        ro, rl = orc.sdpa_fwd(*(x.astype(np.float64) for x in (q[:, h:h + 1], k, v)), is_causal=causal, q_offset=40)
+        assert max_abs(host(o[:, h:h + 1]), ro) <= TOL and lse_rel(host(lse[:, h:h + 1]), rl) <= TOL
