@@ -606,7 +606,10 @@ static MaskSpans mask_spans_plan(const dtattn_prefill_args* a, const dtattn_mask
 // halve the chain of tiles, for 128 KB of LDS at head dim 128 and a merge worth 1-2 us: from 8 tiles on, on grids of one
 // workgroup per CU (causal 1x32/8x1024 22.3 -> 20.9, 777 18.2 -> 16.7, 400 11.9 both; D = 64 1x12x1024 15.8 -> 13.4) and
 // on causal ones of two where the second round is the short blocks of many (1x32/8x1500 32.0 -> 28.8, D = 64 1x12x4096
-// 51.5 -> 39.7; of 7 blocks, 1x64/8x777, 20.1 -> 24.5).
+// 51.5 -> 39.7; of 7 blocks, 1x64/8x777, 20.1 -> 24.5).  A prompt that continues a long context is long rows again: between
+// one and two workgroups per CU (r), the 64-row kernel over this one by the tiles of its first block times r over its
+// blocks: 2.3 to 3.4 1.02-1.12, 4.5 0.96-1.08 (2x32/8x900 behind 1000 keys 52.7 / 55.0), above 0.88-1.02 (3x32/8x512 behind
+// 3000 85 / 96, 4x32/8x512 behind 1000 46.5 / 49.5); with less than 16 tiles in the first block 0.99-1.17.
 static int key_groups(const PrefillParams& p, int D, bool causal, hipStream_t stream) {
     int dev = 0;
     dtattn_device_peaks pk;
@@ -617,7 +620,11 @@ static int key_groups(const PrefillParams& p, int D, bool causal, hipStream_t st
     const int64_t tiles = (keys + 63) / 64;
     if (grid <= pk.cu_count) return tiles >= 8 ? 2 : 1;
     if (grid <= 2 * pk.cu_count) {
-        if (causal) return tiles >= 8 && blocks >= 12 ? 2 : 1;
+        if (causal) {
+            const int64_t first = (std::max<int64_t>(0, std::min<int64_t>(p.Sk, 128 + p.delta)) + 63) / 64;  // tiles of rows 0..127
+            if (D == 128 && first >= 16 && 2 * first * grid >= 9 * blocks * pk.cu_count) return 0;
+            return tiles >= 8 && blocks >= 12 ? 2 : 1;
+        }
         if (tiles <= (p.group >= 4 && p.group % 4 == 0 ? 13 : 16)) return 1;
     }
     return D == 128 ? 0 : 1;

@@ -47,3 +47,24 @@ def test_small_grids(Sq, Sk, D, causal, q_off, k_off, scale, peak, dtype):
     torch.cuda.synchronize()
     assert max_abs(host(o), ro) <= O_TOL_BF16 and lse_rel(host(lse), rl) <= LSE_TOL
     assert max_abs(host(o[0]), host(ob[n - 1])) <= O_TOL_BF16 and lse_rel(host(lse[0]), host(lb[n - 1])) <= 1e-5
+
+
+@pytest.mark.parametrize("D,Sq,before,r", [
+    (128, 300, 900, 1.5), (128, 300, 800, 1.5),      # either side of the rule: 15 and 16 tiles in the first block
+    (128, 1536, 1000, 1.2), (128, 1536, 3000, 1.2),  # two key groups, and the 64-row kernel
+    (64, 300, 1000, 1.5),
+])
+def test_prompts_that_continue_a_context(D, Sq, before, r):
+    """Causal with the diagonal behind `before` keys, on grids of r 128-row workgroups per CU: some heads against the oracle."""
+    import dtorch_amd.nn.functional as F
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.default_rng(Sq + before)
+    H, Sk = int(r * cus) // ((Sq + 127) // 128) // 4 * 4, Sq + before
+    q, k, v = randn(rng, (1, H, Sq, D)), randn(rng, (1, H // 4, Sk, D)), randn(rng, (1, H // 4, Sk, D))
+    tq, tk, tv = (torch.from_numpy(x).to(torch.bfloat16).cuda() for x in (q, k, v))
+    o, lse = F.scaled_dot_product_attention_with_lse(tq, tk, tv, is_causal=True, enable_gqa=True, q_offset=before)
+    torch.cuda.synchronize()
+    for h in (0, H - 1):
+        ro, rl = orc.sdpa_fwd(*(host(t).astype(np.float64) for t in (tq[:, h:h + 1], tk[:, h // 4:h // 4 + 1], tv[:, h // 4:h // 4 + 1])),
+                              is_causal=True, q_offset=before)
+        assert max_abs(host(o[:, h:h + 1]), ro) <= O_TOL_BF16 and lse_rel(host(lse[:, h:h + 1]), rl) <= LSE_TOL
