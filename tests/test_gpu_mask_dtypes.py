@@ -73,7 +73,9 @@ def test_mask_dtypes(dtype, L, S, D, causal, start, pitch):
     (torch.bfloat16, 2, 4, 130, 97, 64, True),
     (torch.float16, 2, 4, 77, 200, 128, False),
     (torch.bfloat16, 8, 8, 1024, 1501, 128, True),   # one row for all queries: read once into fp32 rows
-    (torch.bfloat16, 1, 2, 33, 70, 256, False),      # wide heads: converted first
+    (torch.float16, 8, 8, 1024, 1501, 128, False),
+    (torch.bfloat16, 16, 8, 1024, 1501, 64, False),  # a large row without spans: converted first
+    (torch.bfloat16, 1, 2, 33, 70, 256, False),      # wide heads: likewise
     (torch.float32, 1, 2, 90, 100, 64, False),       # key-split fp32 form
     (torch.float32, 4, 192, 200, 300, 64, True),     # 128-row fp32 form
 ])
